@@ -142,17 +142,21 @@ def _kernel(op, shape, dtype, causal):
     raise refused or RuntimeError(f"no configuration for {operator.describe()}")
 
 
-def prepare(case, seed):
+def _inputs(case, seed):
     op, shape, dtype = case["op"], _shape(case), case["dtype"]
-    operator, kernel = _kernel(op, shape, dtype, bool(case.get("causal", False)))
     if op == "GEMM":
-        inputs = gemm_bench.make_inputs(*shape, seed=seed, dtype=getattr(torch, dtype))
-    elif op == "flash_attn":
-        inputs = attn_bench.make_qkv(*shape, seed=seed)
-    else:
-        # logits spread wider than normalised activations
-        inputs = rowwise_bench.make_inputs(op, *shape, dtype, seed=seed,
-                                           std=2.0 if op == "softmax" else 1.0)
+        return gemm_bench.make_inputs(*shape, seed=seed, dtype=getattr(torch, dtype))
+    if op == "flash_attn":
+        return attn_bench.make_qkv(*shape, seed=seed)
+    # logits spread wider than normalised activations
+    return rowwise_bench.make_inputs(op, *shape, dtype, seed=seed,
+                                     std=2.0 if op == "softmax" else 1.0)
+
+
+def prepare(case, seed):
+    operator, kernel = _kernel(case["op"], _shape(case), case["dtype"],
+                               bool(case.get("causal", False)))
+    inputs = _inputs(case, seed)
     out = operator.make_output(inputs)
     return {"kernel": kernel, "args": operator.kernel_args(inputs, out), "out": out}
 
@@ -185,3 +189,28 @@ def tolerance(case):
     if case["dtype"] == "bfloat16":
         return {"rel": 1e-2, "max": 3.2e-2}
     return {"rel": 1.2e-3, "max": 2.4e-2}
+
+
+def exact(case, seed):
+    """The operator in 64 bits, from torch alone."""
+    inputs = [t.double() for t in _inputs(case, seed)]
+    if case["op"] == "GEMM":
+        a, b = inputs
+        return a @ b
+    if case["op"] == "softmax":
+        return torch.softmax(inputs[0], -1)
+    if case["op"] == "rmsnorm":
+        x, w = inputs
+        return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w
+    q, k, v = inputs
+    out = torch.empty_like(q)
+    hidden = None
+    if case["causal"]:
+        hidden = torch.ones(q.shape[2], k.shape[2], dtype=torch.bool, device=q.device).triu_(1)
+    for b in range(q.shape[0]):
+        for h in range(q.shape[1]):
+            s = (q[b, h] @ k[b, h].t()) * (1.0 / math.sqrt(q.shape[3]))
+            if hidden is not None:
+                s.masked_fill_(hidden, -math.inf)
+            out[b, h] = torch.softmax(s, -1) @ v[b, h]
+    return out
