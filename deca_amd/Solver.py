@@ -506,4 +506,41 @@ def solve_flash_attn(arch, B: int, H: int, S_q: int, S_kv: int, D: int, type_siz
         if int(pipe) == 0 and st >= 2:
             forms += [replace(f, trust=True) for f in forms]
         results += forms
+    return results + _split_forms(arch, B, H, S_q, S_kv, D)
+
+
+# Rows of 32 queries per CU up to which the key-split forms are offered: measured against the
+# plain forms, they win below about 4 (full: 3.9x at 1 row per CU of S = 8192, 1.8x at 2,
+# 1.2x at 2.25, 0.7x at 4) and below about 8 under the causal mask (1.9x at 1, 1.5x at 3,
+# 1.1x at 4, 1.3x at 5.75, whose longest rows no other work hides).
+SPLIT_MAX_ROWS_PER_CU = 8
+
+
+def _split_forms(arch, B: int, H: int, S_q: int, S_kv: int, D: int):
+    """Attention configs whose waves split the keys of one set of query rows (`kv_split`): for
+    grids that leave SIMDs without a wave of query rows of their own.  Of the forms measured on
+    twelve such shapes these were ahead: 32-key tiles on 32x32x16 instructions, one K and one V
+    slot per wave (two at D = 64, with the tile's max not looked at first), and 64 query rows
+    at D = 64."""
+    from deca_amd.kernels.flash_attn_hip import (
+        FAConfig, check_config, est_regs_per_thread, expect_spill_free,
+    )
+
+    if B * H * S_q // 32 >= SPLIT_MAX_ROWS_PER_CU * arch.sm_nums:
+        return []
+    forms = [FAConfig(Br=32, Bc=32, num_warps=nw, stages=st, trust=st > 1, kv_split=True)
+             for nw in (4, 8) for st in ((1, 2) if D <= 64 else (1,))]
+    if D <= 64:
+        forms += [FAConfig(Br=64, Bc=32, num_warps=nw, stages=1, kv_split=True) for nw in (4, 8)]
+    results = []
+    for cfg in forms:
+        try:
+            check_config(cfg, S_q, S_kv, D)
+        except AssertionError:
+            continue
+        regs8 = (est_regs_per_thread(cfg, D) + 7) // 8 * 8
+        waves_per_simd = -(-cfg.num_warps // arch.simds_per_cu)
+        if (expect_spill_free(cfg, D) and regs8 * waves_per_simd <= arch.vgprs_per_simd
+                and (S_q // cfg.Br) * B * H >= arch.sm_nums):
+            results.append(cfg)
     return results

@@ -291,6 +291,44 @@ def fa_occupancy(cfg, arch, D: int, grid: int):
     return wgs, wgs * cfg.num_warps / arch.max_resident_warps_per_sm
 
 
+def fa_split_score(cfg, arch, shape, causal: bool = False) -> float:
+    """Score of a config whose waves share the query rows and split the keys (`kv_split`), on
+    the scale of `fa_score` (useful share of the matrix peak).
+
+    Its time is modelled directly: a fixed part per workgroup (Q, the first tiles, the meeting
+    of the waves in LDS) and a number of key steps per wave whose length grows with the waves
+    that share a SIMD.  Fitted on twelve shapes of 256 ... 2048 rows of 32 queries (S = 512 ...
+    16384, D = 64 and 128, full and causal), where it is within 10 % of the measured time of
+    these forms.  `fa_score` overestimates the plain forms on such small grids, more so under
+    the causal mask (their measured times are 1.05x and 1.35x its own at the median), hence
+    the last factor."""
+    B, H, S_q, S_kv, D = shape
+    grid = (S_q // cfg.Br) * B * H
+    wgs, _ = fa_occupancy(cfg, arch, D, grid)
+    per_cu = min(wgs, math.ceil(grid / arch.sm_nums))
+
+    def key_step(workgroups):
+        waves = max(1.0, workgroups * cfg.num_warps / arch.simds_per_cu)
+        # a second slot per wave pays while a tile is small (D = 64: -7 %; D = 128: +7 %)
+        slots = 1.0 if cfg.stages == 1 else (0.93 if cfg.Bc * D <= 32 * 64 else 1.07)
+        return (0.25e-6 + 0.65e-6 * waves * (cfg.Br // 32)) * (cfg.Bc / 32) * (D / 128) * slots
+
+    step = key_step(per_cu)
+    fixed, launch = 3.3e-6, 1.5e-6  # per workgroup; of the first one, what every launch costs
+    steps = math.ceil(S_kv / (cfg.Bc * cfg.num_warps))
+    longest = fixed + steps * step
+    rounds = grid / (arch.sm_nums * wgs)
+    if causal:
+        # (the longest workgroups start first and are alone on their CU towards the end)
+        longest = fixed + steps * 0.5 * (step + key_step(1))
+        mean = fixed + (S_kv / 2 + cfg.Br / 2) / (cfg.Bc * cfg.num_warps) * step
+        t = max(longest, rounds * mean)
+    else:
+        t = math.ceil(rounds) * longest
+    flops = 4.0 * B * H * S_q * S_kv * D * (0.5 if causal else 1.0)
+    return flops / (arch.peak_mma_sync_flops * 1e9) / ((t - launch) * (0.8 if causal else 0.95))
+
+
 def fa_score(cfg, arch, shape, causal: bool = False) -> float:
     """
     Heuristic score of a FlashAttention config.
@@ -309,6 +347,8 @@ def fa_score(cfg, arch, shape, causal: bool = False) -> float:
     - causal: tiles crossing the diagonal are computed in full, so only the
       useful fraction of the computed score tiles counts
     """
+    if getattr(cfg, "kv_split", False):
+        return fa_split_score(cfg, arch, shape, causal)
     B, H, S_q, S_kv, D = shape
     grid = (S_q // cfg.Br) * B * H
     wgs, _ = fa_occupancy(cfg, arch, D, grid)

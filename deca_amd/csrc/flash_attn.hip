@@ -20,6 +20,15 @@
 //   DECA_TRUST          1 (plain ring loops): a tile's exponentials are taken against the
 //                       running max as it stands, without looking at the tile's own max
 //                       first; a tile that turns out to have outgrown it is done again
+//   DECA_KVSPLIT        1 (plain loop): the waves of a workgroup share its query rows and
+//                       take the key tiles in turn, each through an LDS ring of its own
+//                       and without barriers; their results meet in LDS at the end
+//                       Why: a grid of few query rows is bound by what one wave can do in
+//                       series, with three SIMDs of a CU idle (B1 H16 S_q 512 S_kv 8192
+//                       D 128: 256 rows of 32 queries, 185 us at one wave each, 49 us with
+//                       eight; S_q = S_kv = 512, D 64, causal: 9.9 and 5.2 us).  Bound
+//                       then: the CU's load path, which streams all K/V of a row (4 MiB at
+//                       64 B/clk: 28 us of the 49).
 //   DECA_CAUSAL         1: key j visible to query i iff j <= i (SQ == SKV)
 //   DECA_SCALE          softmax scale
 //   DECA_PIPE           1: S^T of the next tile is computed before the softmax of
@@ -92,6 +101,9 @@
 #ifndef DECA_TRUST
 #define DECA_TRUST 0
 #endif
+#ifndef DECA_KVSPLIT
+#define DECA_KVSPLIT 0
+#endif
 // In the 16x16x32 form the plain loops take a tile's row sums on the matrix pipe (one more
 // product per k-step, with a ones operand: four accumulator registers per query tile), which
 // frees the vector ALU of one add per score; l is then the sum of the fp16 P that the second
@@ -106,7 +118,8 @@
 #endif
 
 constexpr int NT = NW * 64;
-constexpr int WQ = BR / NW;       // query rows per wave
+constexpr int WQ = DECA_KVSPLIT ? BR : BR / NW;  // query rows per wave
+constexpr int KVG = DECA_KVSPLIT ? NW : 1;       // waves that share the keys of one query row
 #ifndef DECA_MFMA16
 #define DECA_MFMA16 0  // 1: v_mfma_f32_16x16x32_f16 tiles (plain loop only) instead of 32x32x16
 #endif
@@ -139,20 +152,33 @@ constexpr int K_CHUNKS_PER_STEP = 2, V_CHUNKS_PER_BLOCK = 4;
 constexpr int CPR = D_ / 8;       // 16-byte chunks per K/V row
 constexpr int TILE_CHUNKS = BC * CPR;
 constexpr int TILE_BYTES = TILE_CHUNKS * 16;
-constexpr int KV_IT = TILE_CHUNKS / NT;
+constexpr int KV_NT = NT / KVG;   // lanes that bring in one K/V tile
+constexpr int KV_IT = TILE_CHUNKS / KV_NT;
 constexpr int NKV = DECA_SKV / BC;
-constexpr int RING_BYTES = 2 * STAGES * TILE_BYTES;
+constexpr int RING_BYTES = 2 * STAGES * TILE_BYTES;      // (one ring per wave with DECA_KVSPLIT)
 constexpr int Q_LDS_OFFSET = RING_BYTES;                 // the Q tile follows the K/V ring
-constexpr int LDS_BYTES = RING_BYTES + (DECA_QSMEM ? BR * D_ * 2 : 0);
+// DECA_KVSPLIT, after the loop: every wave's O^T accumulators as OUNITS runs of 1 KiB (one
+// floatx4 per lane), then its running max and row sum per query tile.
+constexpr int OUNITS = DT * MQ * (ACC_N / 4);
+constexpr int PART_BYTES = NW * OUNITS * 1024;
+constexpr int COMBINE_BYTES = DECA_KVSPLIT ? PART_BYTES + NW * MQ * 512 : 0;
+constexpr int LOOP_BYTES = KVG * RING_BYTES + (DECA_QSMEM ? BR * D_ * 2 : 0);
+constexpr int LDS_BYTES = LOOP_BYTES > COMBINE_BYTES ? LOOP_BYTES : COMBINE_BYTES;
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float NEG_INF = -1e30f;
+// The running max before the first tile.  A wave that takes every tile of a causal row sees
+// key 0 first; one that takes a share of them may meet a tile whose keys are all masked for
+// some row: from a start far above the mask value (and far below any score) their p are 0
+// and the row's max, sum and O stay as they started.
+constexpr float M_START = DECA_KVSPLIT ? -1e28f : NEG_INF;
 constexpr float SL2 = static_cast<float>(DECA_SCALE) * LOG2E;
 
 static_assert(D_ % 64 == 0 && D_ >= 64, "head dim: a multiple of 64 (flash_attn_tir.py:70-72)");
-static_assert(BR % (32 * NW) == 0, "each wave owns a multiple of 32 query rows");
+static_assert(WQ % 32 == 0 && BR % WQ == 0, "each wave owns a multiple of 32 query rows");
+static_assert(!DECA_KVSPLIT || (DECA_PIPE == 0 && !DECA_QSMEM && NW >= 2), "key split: plain loop, Q in registers");
 static_assert(BC % 32 == 0, "BC must be a multiple of 32");
 static_assert(DECA_SQ % BR == 0 && DECA_SKV % BC == 0, "tiles must divide the sequences");
-static_assert(TILE_CHUNKS % NT == 0, "loader coverage");
+static_assert(TILE_CHUNKS % KV_NT == 0, "loader coverage");
 static_assert(STAGES >= 1 && STAGES <= 3, "K/V ring depth");
 static_assert(STAGES < 3 || DECA_PIPE == 0, "three stages: plain loop only");
 static_assert(!DECA_TRUST || (DECA_PIPE == 0 && STAGES >= 2), "trust: a form of the plain ring loops");
@@ -301,6 +327,11 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  // Which WQ rows of the workgroup's tile this wave owns, and which share of the keys: key
+  // tile j of the wave is tile j * KVG + kvg of the sequence.
+  const int qw = DECA_KVSPLIT ? 0 : wave;
+  const int qw_u = DECA_KVSPLIT ? 0 : wave_u;
+  const int kvg = DECA_KVSPLIT ? wave_u : 0;
   const int l32 = lane & 31;
   const int half = lane >> 5;
   // ---- workgroup -> (batch*head, query tile) ------------------------------------------
@@ -332,25 +363,29 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     bh = blockIdx.x % BH;
     qt = (NQ - 1) - blockIdx.x / BH;
   }
-  const int nkv = ((qt + 1) * BR + BC - 1) / BC;
+  const int nkv_all = ((qt + 1) * BR + BC - 1) / BC;
 #else
   int lin = blockIdx.x;
   if (TOTAL % 8 == 0) lin = (lin & 7) * (TOTAL / 8) + (lin >> 3);
   const int bh = lin / NQ;
   const int qt = lin % NQ;
-  const int nkv = NKV;
+  const int nkv_all = NKV;
 #endif
-  const _Float16* q_base = Q + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + wave * WQ) * D_;
-  const _Float16* k_base = K + static_cast<size_t>(bh) * DECA_SKV * D_;
-  const _Float16* v_base = V + static_cast<size_t>(bh) * DECA_SKV * D_;
-  _Float16* o_base = O + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + wave * WQ) * D_;
+  const int nkv = (nkv_all - kvg + KVG - 1) / KVG;  // (a wave's share may be empty)
+  const _Float16* q_base = Q + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + qw * WQ) * D_;
+  const _Float16* k_base = K + static_cast<size_t>(bh) * DECA_SKV * D_ + kvg * (BC * D_);
+  const _Float16* v_base = V + static_cast<size_t>(bh) * DECA_SKV * D_ + kvg * (BC * D_);
+  _Float16* o_base = O + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + qw * WQ) * D_;
 
   // ---- K/V tile loads: global -> LDS, asynchronous ------------------------------
-  const unsigned lds_u = static_cast<unsigned>(reinterpret_cast<size_t>((lptr)lds));
+  const unsigned lds_u = static_cast<unsigned>(reinterpret_cast<size_t>((lptr)lds)) + kvg * RING_BYTES;
+  const int kv_wave = DECA_KVSPLIT ? 0 : wave_u;  // wave and lane among those that bring in a tile
+  const int kv_tid = DECA_KVSPLIT ? lane : tid;
+  constexpr size_t KV_STRIDE = static_cast<size_t>(KVG) * BC * D_;  // elements between a wave's tiles
   unsigned k_voff[KV_IT], v_voff[KV_IT];
 #pragma unroll
   for (int it = 0; it < KV_IT; ++it) {
-    const int sidx = it * NT + tid;
+    const int sidx = it * KV_NT + kv_tid;
     const int row = sidx / CPR, cs = sidx % CPR;
     const int ck = cs ^ k_swz(row);
     const int cv = cs ^ v_swz(row);
@@ -366,16 +401,16 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                  : "memory", "m0");
   };
   auto issue_k = [&](int j, int slot) __attribute__((always_inline)) {
-    const _Float16* origin = k_base + static_cast<size_t>(j) * BC * D_;
-    const unsigned dst = lds_u + slot * TILE_BYTES + wave_u * 1024;
+    const _Float16* origin = k_base + j * KV_STRIDE;
+    const unsigned dst = lds_u + slot * TILE_BYTES + kv_wave * 1024;
 #pragma unroll
-    for (int it = 0; it < KV_IT; ++it) dma16(origin, k_voff[it], dst + it * NT * 16);
+    for (int it = 0; it < KV_IT; ++it) dma16(origin, k_voff[it], dst + it * KV_NT * 16);
   };
   auto issue_v = [&](int j, int slot) __attribute__((always_inline)) {
-    const _Float16* origin = v_base + static_cast<size_t>(j) * BC * D_;
-    const unsigned dst = lds_u + (STAGES + slot) * TILE_BYTES + wave_u * 1024;
+    const _Float16* origin = v_base + j * KV_STRIDE;
+    const unsigned dst = lds_u + (STAGES + slot) * TILE_BYTES + kv_wave * 1024;
 #pragma unroll
-    for (int it = 0; it < KV_IT; ++it) dma16(origin, v_voff[it], dst + it * NT * 16);
+    for (int it = 0; it < KV_IT; ++it) dma16(origin, v_voff[it], dst + it * KV_NT * 16);
   };
 
   // Load number l of the 2 * KV_IT that bring in tile j (K chunks first, then V), and the
@@ -385,11 +420,11 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   auto issue_kv_load = [&](int jk, int kslot, int jv, int vslot, int l) __attribute__((always_inline)) {
     if (l < KV_IT) {
       if (jk < nkv)
-        dma16(k_base + static_cast<size_t>(jk) * BC * D_, k_voff[l],
-              lds_u + kslot * TILE_BYTES + wave_u * 1024 + l * NT * 16);
+        dma16(k_base + jk * KV_STRIDE, k_voff[l],
+              lds_u + kslot * TILE_BYTES + kv_wave * 1024 + l * KV_NT * 16);
     } else {
-      dma16(v_base + static_cast<size_t>(jv) * BC * D_, v_voff[l - KV_IT],
-            lds_u + (STAGES + vslot) * TILE_BYTES + wave_u * 1024 + (l - KV_IT) * NT * 16);
+      dma16(v_base + jv * KV_STRIDE, v_voff[l - KV_IT],
+            lds_u + (STAGES + vslot) * TILE_BYTES + kv_wave * 1024 + (l - KV_IT) * KV_NT * 16);
     }
   };
   auto issue_kv_share = [&](int jk, int kslot, int jv, int vslot, int i, int n) __attribute__((always_inline)) {
@@ -417,7 +452,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     constexpr int Q_IT = WQ * CPR / 64;
     static_assert((WQ * CPR) % 64 == 0, "a wave's Q rows are whole 1 KiB runs");
     const unsigned dst = lds_u + Q_LDS_OFFSET + wave_u * (WQ * D_ * 2);
-    const _Float16* q_origin = Q + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + wave_u * WQ) * D_;
+    const _Float16* q_origin = Q + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + qw_u * WQ) * D_;
 #pragma unroll
     for (int it = 0; it < Q_IT; ++it) {
       const int sidx = it * 64 + lane;
@@ -445,7 +480,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   float m_i[MQ], l_i[MQ];
 #pragma unroll
   for (int mq = 0; mq < MQ; ++mq) {
-    m_i[mq] = NEG_INF;
+    m_i[mq] = M_START;
     l_i[mq] = 0.0f;
   }
 
@@ -456,7 +491,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   // K: row = kt*32 + lane%32, chunk = (ks*2 + half) ^ k_swz(row); the row bits used by
   // the swizzle do not depend on kt (k_swz has period 16).
   // (16x16x32: row = kt*16 + lane%16, chunk = (ks*4 + lane/16) ^ k_swz(row))
-  unsigned k_lane_base = static_cast<unsigned>(lq * CPR + (lg ^ k_swz(lq))) * 16u;
+  unsigned k_lane_base = static_cast<unsigned>(lq * CPR + (lg ^ k_swz(lq))) * 16u + static_cast<unsigned>(kvg) * RING_BYTES;
   auto k_frag_offset = [&](int ks, int kt) __attribute__((always_inline)) {
     return (k_lane_base ^ k_xor_const(ks * K_CHUNKS_PER_STEP)) + k_add_const(ks * K_CHUNKS_PER_STEP) +
            static_cast<unsigned>(kt * TQ * CPR * 16);
@@ -481,7 +516,8 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
 #endif
   const unsigned v_lane_base = static_cast<unsigned>(
       v_row0 * CPR * 16 + (((v_d0 >> 3) ^ v_swz(v_row0)) * 16) +
-      ((v_d0 >> 2) & 1) * 8);
+      ((v_d0 >> 2) & 1) * 8) + static_cast<unsigned>(kvg) * RING_BYTES;
+  static_assert(RING_BYTES % 256 == 0, "the XOR constants reach address bits 4..7 only");
   static_assert(CPR >= 8, "D >= 64");
   auto v_frag_offset = [&](int dt, int row0) __attribute__((always_inline)) {
     return (v_lane_base ^ v_xor_const(dt * V_CHUNKS_PER_BLOCK)) + v_add_const(dt * V_CHUNKS_PER_BLOCK) +
@@ -512,24 +548,26 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
       }
     }
   };
+  // first key of this wave's tile j
+  auto key0 = [&](int j) __attribute__((always_inline)) { return (j * KVG + kvg) * BC; };
   auto nothing = [](int) __attribute__((always_inline)) {};
   // Causal mask of tile j.  Only tiles crossing the diagonal need it; every
   // query sees key 0 in tile 0, so its running max is finite before a fully
   // masked block shows up.
   auto mask_s = [&](acc_t (&s_acc)[KT][MQ], int j) __attribute__((always_inline)) {
 #if DECA_CAUSAL
-    if ((j + 1) * BC - 1 > qt * BR + wave * WQ) {
+    if (key0(j) + BC - 1 > qt * BR + qw * WQ) {
 #pragma unroll
       for (int mq = 0; mq < MQ; ++mq) {
-        const int q_idx = qt * BR + wave * WQ + mq * TQ + lq;
+        const int q_idx = qt * BR + qw * WQ + mq * TQ + lq;
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
           for (int e = 0; e < ACC_N; ++e) {
 #if DECA_MFMA16
-            const int kv_idx = j * BC + kt * 16 + lg * 4 + e;
+            const int kv_idx = key0(j) + kt * 16 + lg * 4 + e;
 #else
-            const int kv_idx = j * BC + kt * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
+            const int kv_idx = key0(j) + kt * 32 + (e >> 2) * 8 + half * 4 + (e & 3);
 #endif
             if (kv_idx > q_idx) s_acc[kt][mq][e] = NEG_INF;
           }
@@ -758,7 +796,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   auto wait_and_barrier = [&]() __attribute__((always_inline)) {
     DECA_WAIT_VMCNT(0);                  // this lane's outstanding tile loads have landed
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's LDS reads have returned
-    __builtin_amdgcn_s_barrier();
+    if (!DECA_KVSPLIT) __builtin_amdgcn_s_barrier();  // (a ring of the wave's own owes none)
     asm volatile("" ::: "memory");       // no LDS read of the new tile moves above the barrier
   };
 
@@ -775,7 +813,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     else
       DECA_WAIT_VMCNT(0);
     __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_s_barrier();
+    if (!DECA_KVSPLIT) __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     const int ahead = j + 2;                        // the tile this step requests ...
     const int fill = slot == 0 ? 2 : slot - 1;      // ... and the ring slot it goes to
@@ -794,7 +832,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     // there is nothing to add.  (Skipping single masked 32-key blocks of the
     // diagonal tiles as well was tried: the extra code paths cost registers and
     // made the kernel slower.)
-    const bool skip = j * BC > qt * BR + wave_u * WQ + WQ - 1;
+    const bool skip = key0(j) > qt * BR + qw_u * WQ + WQ - 1;
 #else
     const bool skip = false;
 #endif
@@ -813,7 +851,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     bool in_full = j == 0;
 #if DECA_CAUSAL
     // a tile that reaches the diagonal for this wave needs the mask: never on trust
-    in_full |= (j + 1) * BC - 1 > qt * BR + wave_u * WQ;
+    in_full |= key0(j) + BC - 1 > qt * BR + qw_u * WQ;
 #endif
     bool request = more;  // the next tile's loads ride on the first pass only
 #pragma unroll 1
@@ -1236,7 +1274,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   wait_and_barrier();
 #if DECA_CAUSAL
   // (unless every key of it lies after every query row of this wave: P = 0 exactly)
-  if ((nkv - 1) * BC <= qt * BR + wave_u * WQ + WQ - 1)
+  if ((nkv - 1) * BC <= qt * BR + qw_u * WQ + WQ - 1)
 #endif
   {
     rescale_o();
@@ -1245,8 +1283,10 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   }
 #endif
 #else
-  issue_k(0, 0);
-  issue_v(0, 0);
+  if (!DECA_KVSPLIT || nkv > 0) {
+    issue_k(0, 0);
+    issue_v(0, 0);
+  }
 #if STAGES == 3
   if (nkv > 1) {
     issue_k(1, 1);
@@ -1271,6 +1311,33 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     kv_step(j, 0);
     if (j + 1 < nkv) kv_step(j + 1, 1);
   }
+#elif DECA_KVSPLIT
+  // One K and one V slot, both the wave's own: K_{j+1} is requested as soon as S^T of tile j
+  // has read K_j, V_{j+1} as soon as O^T has read V_j, so each has the other half of a step
+  // to land.  Loads return in order and K_j is older than V_j: what may stay outstanding in
+  // front of either product is the one tile requested after it.
+  for (int j = 0; j < nkv; ++j) {
+    const bool more = j + 1 < nkv;
+    DECA_WAIT_VMCNT(KV_IT);
+    asm volatile("" ::: "memory");
+    acc_t s_acc[KT][MQ];
+    half8 pf[KK][MQ];
+    compute_s(s_acc, 0, nothing);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of K_j have returned
+    asm volatile("" ::: "memory");
+    if (more) issue_k(j + 1, 0);
+    mask_s(s_acc, j);
+    softmax(s_acc, pf);
+    if (more)
+      DECA_WAIT_VMCNT(KV_IT);
+    else
+      DECA_WAIT_VMCNT(0);
+    asm volatile("" ::: "memory");
+    compute_pv(pf, 0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("" ::: "memory");
+    if (more) issue_v(j + 1, 0);
+  }
 #else
   for (int j = 0; j < nkv; ++j) {
     wait_and_barrier();
@@ -1291,6 +1358,63 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
 #endif
 #endif
 
+#if DECA_KVSPLIT
+  // ---- epilogue: the waves' shares of the keys become one row -------------------------------
+  // Wave g holds, for all of its queries, max m_g, sum l_g and O^T_g over its share; with
+  // M = max m_g and w_g = exp2((m_g - M) * sl2), O = sum w_g O_g / sum w_g l_g.  Everything
+  // stays in fp32 and goes through LDS once; each wave then finishes 1 / NW of the row.
+  {
+    floatx4* part = reinterpret_cast<floatx4*>(lds);
+    float* stat = reinterpret_cast<float*>(lds + PART_BYTES);  // [NW][MQ][max, sum][64]
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __syncthreads();  // every wave is done reading its K/V ring
+    constexpr int QUADS = ACC_N / 4;
+#pragma unroll
+    for (int mq = 0; mq < MQ; ++mq) {
+#if DECA_MFMASUM
+      const float l = l_i[mq];
+#else
+      const float l = sum_over_query(l_i[mq]);
+#endif
+      stat[(wave * MQ + mq) * 128 + lane] = m_i[mq];
+      stat[(wave * MQ + mq) * 128 + 64 + lane] = l;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < QUADS; ++g) {
+          floatx4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = o_acc[dt][mq][g * 4 + e];
+          part[((wave * DT + dt) * MQ + mq) * QUADS * 64 + g * 64 + lane] = v;
+        }
+    }
+    __syncthreads();
+    for (int u = wave_u; u < OUNITS; u += NW) {
+      const int g = u % QUADS, mq = u / QUADS % MQ, dt = u / (QUADS * MQ);
+      float m[NW], top = M_START;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        m[i] = stat[(i * MQ + mq) * 128 + lane];
+        top = fmaxf(top, m[i]);
+      }
+      float l = 0.0f;
+      floatx4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        const float w = __builtin_amdgcn_exp2f((m[i] - top) * SL2);
+        l += w * stat[(i * MQ + mq) * 128 + 64 + lane];
+        const floatx4 v = part[(i * OUNITS + u) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += w * v[e];
+      }
+      const float inv = 1.0f / l;
+      half4 h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(o[e] * inv);
+      *reinterpret_cast<half4*>(o_base + (mq * TQ + lq) * D_ + lg * 4 + dt * TQ + g * 8) = h;
+    }
+  }
+#else
   // ---- epilogue: O[q][d] = O^T[d][q] / l ----------------------------------------------
   // o_acc[dt][mq][e]: q = mq*32 + lane%32, d = dt*32 + (e/4)*8 + half*4 + e%4.
   // A lane owns 8-byte pieces of a row; when the K/V ring is large enough the
@@ -1338,4 +1462,5 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
       *reinterpret_cast<u32x4*>(o_base + row * D_ + c * 8) = v;
     }
   }
+#endif  // DECA_KVSPLIT
 }

@@ -71,6 +71,16 @@ class FAConfig:
     # first one always takes its max) is computed again with it.  Same quotient O / l.
     # Measured: +3.6 % at D = 64 and D = 128 (S = 4096, full); nothing with the causal mask.
     trust: bool = False
+    # Plain loop: the waves of a workgroup all own its Br query rows and take the key tiles in
+    # turn, each through an LDS ring of its own and without barriers in the loop; their
+    # maxima, sums and O^T meet in LDS at the end.  For grids with too few query rows to give
+    # every SIMD a wave of its own.
+    kv_split: bool = False
+
+    @property
+    def wave_rows(self) -> int:
+        """Query rows of one wave."""
+        return self.Br if self.kv_split else self.Br // self.num_warps
 
     @property
     def threads(self) -> int:
@@ -88,6 +98,7 @@ class FAConfig:
             + (",roll=1" if self.roll else "")
             + (f",spread={self.spread}" if self.spread else "")
             + (",trust=1" if self.trust else "")
+            + (",kvs=1" if self.kv_split else "")
         )
 
 
@@ -103,13 +114,18 @@ def default_spread(cfg: FAConfig) -> int:
 
 def smem_bytes(cfg: FAConfig, D: int) -> int:
     """`stages` K tiles and `stages` V tiles of Bc x D halves, and the Q tile when it is
-    staged (flash_attn_tir.py:54-56; rows are never padded here)."""
+    staged (flash_attn_tir.py:54-56; rows are never padded here).  With `kv_split` every wave
+    has a ring, and afterwards its fp32 O^T, row maxima and row sums in their place."""
+    if cfg.kv_split:
+        ring = 2 * cfg.stages * cfg.Bc * D * 2
+        query_tiles = cfg.Br // (16 if cfg.mfma == 16 else 32)
+        return cfg.num_warps * max(ring, cfg.Br * D * 4 + query_tiles * 512)
     return (2 * cfg.stages * cfg.Bc + (cfg.Br if cfg.q_in_smem else 0)) * D * 2
 
 
 def est_regs_per_thread(cfg: FAConfig, D: int) -> int:
     """Unified VGPR estimate per lane of the live fragments."""
-    mq = cfg.Br // cfg.num_warps // 32
+    mq = cfg.wave_rows // 32
     o_acc = (D // 32) * mq * 16
     s_acc = (cfg.Bc // 32) * mq * 16
     p_h = s_acc // 2
@@ -188,16 +204,19 @@ def check_config(cfg: FAConfig, S_q: int, S_kv: int, D: int) -> None:
     # as the reference (flash_attn_tir.py:70-72); the LDS swizzles only touch the low chunk
     # bits of a row, so any row of a multiple of 8 chunks works
     assert D % 64 == 0 and D >= 64, "head dim must be a multiple of 64"
-    assert cfg.Br % (32 * cfg.num_warps) == 0
+    assert cfg.Br % 32 == 0 and (cfg.kv_split or cfg.Br % (32 * cfg.num_warps) == 0)
+    assert not cfg.kv_split or (int(cfg.pipe) == 0 and not cfg.q_in_smem and cfg.num_warps >= 2), \
+        "the key split is a form of the plain loop with Q in registers"
     assert cfg.Bc % 32 == 0
     assert S_q % cfg.Br == 0 and S_kv % cfg.Bc == 0
     cpr = D // 8
-    assert (cfg.Bc * cpr) % cfg.threads == 0
-    assert 2 * (cfg.Bc * cpr) // cfg.threads <= 63
+    loaders = WAVE if cfg.kv_split else cfg.threads  # lanes that bring in one K/V tile
+    assert (cfg.Bc * cpr) % loaders == 0
+    assert 2 * (cfg.Bc * cpr) // loaders <= 63
     assert cfg.threads <= 1024
     assert cfg.stages in (1, 2, 3)
     assert cfg.stages < 3 or int(cfg.pipe) == 0, "three stages: plain loop only"
-    assert cfg.stages < 3 or 4 * (cfg.Bc * cpr) // cfg.threads <= 63
+    assert cfg.stages < 3 or 4 * (cfg.Bc * cpr) // loaders <= 63
     assert int(cfg.pipe) in (0, 1, 2)
     assert cfg.mfma in (32, 16)
     assert cfg.mfma == 32 or int(cfg.pipe) != 1, "the 16x16x32 form exists for the plain and the slot loop"
@@ -251,13 +270,16 @@ def make_flash_attn_fwd(
         defines["DECA_SPREAD"] = cfg.spread
     if cfg.trust:
         defines["DECA_TRUST"] = 1
-    # The three-stage ring waits for part of its outstanding loads, which is only right
+    if cfg.kv_split:
+        defines["DECA_KVSPLIT"] = 1
+    # The three-stage ring, and the one-stage ring of a wave's own (`kv_split`), wait for part
+    # of their outstanding loads, which is only right
     # while the tile loads are the loop's only vector-memory traffic: a build that spills
     # (scratch stores share the counter and retire out of order) is refused at load time.
     return make_spec(
         TEMPLATE, defines, grid=((S_q // cfg.Br) * B * H, 1, 1), block=(cfg.threads, 1, 1), nargs=4,
         options=FAST_MATH_OPTIONS,
-        meta={"cfg": str(cfg), "causal": causal, "no_scratch": cfg.stages > 2},
+        meta={"cfg": str(cfg), "causal": causal, "no_scratch": cfg.stages > 2 or (cfg.kv_split and cfg.stages == 1)},
     )
 
 

@@ -286,6 +286,24 @@ FA_CASES = [
     (1, 2, 512, 512, 128, False, FAConfig(256, 64, 8, 2, q_in_smem=True, swizzle=False, pipe=2, mfma=16)),
 ]
 
+# the waves of a workgroup share its query rows and take the key tiles in turn: fewer tiles
+# than waves (empty shares), an uneven number of them, causal rows for which a wave's first
+# tile is masked throughout, one to three slots, both tile forms, two query tiles per wave
+FA_SPLIT_CASES = [
+    (1, 2, 64, 64, 64, False, FAConfig(32, 32, 4, 1, kv_split=True)),
+    (1, 2, 32, 96, 128, False, FAConfig(32, 32, 8, 1, kv_split=True)),
+    (1, 3, 96, 672, 128, False, FAConfig(32, 32, 8, 1, kv_split=True)),
+    (1, 2, 256, 256, 128, True, FAConfig(32, 32, 8, 1, kv_split=True)),
+    (1, 2, 288, 288, 64, True, FAConfig(32, 32, 4, 2, trust=True, kv_split=True)),
+    (1, 8, 128, 1056, 64, False, FAConfig(32, 32, 8, 2, trust=True, kv_split=True)),
+    (1, 2, 320, 320, 64, True, FAConfig(64, 32, 8, 1, kv_split=True)),
+    (2, 4, 192, 544, 64, False, FAConfig(64, 32, 4, 1, kv_split=True)),
+    (1, 2, 256, 256, 128, True, FAConfig(32, 64, 4, 1, mfma=16, kv_split=True)),
+    (1, 2, 128, 320, 64, False, FAConfig(64, 64, 2, 3, mfma=16, kv_split=True)),
+    (1, 2, 160, 160, 128, True, FAConfig(32, 32, 2, 2, mfma=16, roll=True, spread=2, trust=True, kv_split=True)),
+    (1, 1, 64, 320, 192, False, FAConfig(32, 32, 4, 1, kv_split=True)),
+]
+
 FA_FULL = [
     (4, 16, 4096, 4096, 128, False, FAConfig(128, 64, 4, 2)),
     (4, 16, 4096, 4096, 128, True, FAConfig(128, 64, 4, 2)),
@@ -307,7 +325,7 @@ FA_FULL = [
 
 def fa_specs():
     return [make_flash_attn_fwd(B, H, Sq, Skv, D, cfg, None, causal)
-            for B, H, Sq, Skv, D, causal, cfg in FA_CASES + FA_FULL]
+            for B, H, Sq, Skv, D, causal, cfg in FA_CASES + FA_SPLIT_CASES + FA_FULL]
 
 
 def spilling_specs():
