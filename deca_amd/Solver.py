@@ -386,7 +386,42 @@ def solve_gemm_tc(arch, M: int, N: int, K: int, type_size: int = 2, count: int =
                     except AssertionError:
                         continue
                 results.append(cand)
+    if results:
+        results += _edge_forms(arch, M, N, K)
     return results[:count]
+
+
+def _edge_forms(arch, M: int, N: int, K: int):
+    """GEMM configs whose workgroup tiles need not divide M and N (`edge`), for shapes that
+    are no multiple of 256 both ways: the eight-wave tile bodies measured on such shapes
+    (`cost_model.GEMM_STEP_TIMES`), in every tile order, down to half a tile per CU.  (A grid
+    of 242 tiles of 128 x 128 is 1.9x faster than 462 of 64 x 128, the best that divide
+    1344 x 2816.)"""
+    from dataclasses import replace
+
+    from deca_amd.cost_model.CostModel import GEMM_STEP_TIMES
+    from deca_amd.kernels.gemm_hip import (
+        GemmConfig, agpr_split_fits, check_config, default_spread, tile_grid,
+    )
+
+    if (M % 256 == 0 and N % 256 == 0) or N % 8:
+        return []
+    results = []
+    for bm, bn, bk, wm, wn, st in GEMM_STEP_TIMES:
+        if K % bk or K // bk < st:
+            continue
+        cfg = GemmConfig(BM=bm, BN=bn, BK=bk, warp_m=wm, warp_n=wn, stages=st, epi_smem=True,
+                         mfma=16, early=wm // 32 if wm >= 64 else 0, edge=True)
+        cfg = replace(cfg, agpr=agpr_split_fits(cfg), spread=default_spread(cfg))
+        rows, cols = tile_grid(cfg, M, N)
+        if 2 * rows * cols < arch.sm_nums:
+            continue
+        for ras in GEMM_RASTERS:
+            if 0 < ras <= rows:
+                cand = replace(cfg, raster=ras)
+                check_config(cand, M, N, K)
+                results.append(cand)
+    return results
 
 
 # ---------------------------------------------------------------------------

@@ -126,7 +126,9 @@ def gemm_wave_dram_bytes_per_flop(cfg, arch, M: int, N: int, K: int, slots: int)
     cache = getattr(arch, "mall_bytes", arch.l2_bytes)
     if (M * K + K * N) * 2 <= 0.5 * cache:
         return (M * K + K * N) * 2 / (2.0 * M * N * K)
-    GM, GN = M // cfg.BM, N // cfg.BN
+    from deca_amd.kernels.gemm_hip import tile_grid
+
+    GM, GN = tile_grid(cfg, M, N)
     if cfg.raster == 0:  # the tiles in flight form 16 x 16 blocks
         blocks = max(1, math.ceil(min(slots, GM * GN) / 256))
         return blocks * 16 * (cfg.BM + cfg.BN) / (min(slots, GM * GN) * cfg.BM * cfg.BN)
@@ -140,6 +142,44 @@ def gemm_wave_dram_bytes_per_flop(cfg, arch, M: int, N: int, K: int, slots: int)
 def gemm_mma_peak(cfg, arch) -> float:
     """MFMA peak (GFLOPS) with fp32 accumulation, the only mode of the matrix cores."""
     return arch.peak_mma_sync_flops
+
+
+# Measured times of the eight-wave tile bodies (16x16x32 tiles, accumulators in AGPRs where
+# they fit, load window): (BM, BN, BK, warp_m, warp_n, stages) -> microseconds of
+# (a workgroup's prologue and epilogue, one K-tile of a workgroup alone on its CU, one K-tile
+# of each of two on a CU).  Fitted to seven shapes that are multiples of 64 and of little else
+# (M 704 ... 4800, N 640 ... 7360, K 512 ... 5440); the times these give are within 10 % there.
+# What they show is the CU's load path and the fabric behind its L2 rather than the matrix pipe:
+# 32 KiB per 128 x 128 K-tile at 70 KB/us and CU.
+GEMM_STEP_TIMES = {
+    (256, 256, 64, 128, 64, 2): (6.0, 1.154, 2.308),
+    (256, 128, 64, 64, 64, 3): (2.6, 0.776, 1.552),
+    (128, 256, 64, 64, 64, 3): (2.7, 0.757, 1.514),
+    (128, 128, 64, 64, 32, 3): (1.3, 0.476, 0.952),
+    (128, 64, 64, 64, 32, 3): (1.0, 0.304, 0.594),
+    (64, 128, 64, 64, 32, 3): (1.0, 0.301, 0.597),
+    (64, 64, 64, 32, 32, 5): (1.0, 0.225, 0.390),
+}
+
+
+def gemm_edge_score(cfg, arch, M: int, N: int, K: int) -> float:
+    """Score of an `edge` config: useful share of the matrix peak in the time that
+    `GEMM_STEP_TIMES` gives it."""
+    from deca_amd.kernels.gemm_hip import tile_grid
+
+    fixed, one, two = GEMM_STEP_TIMES[(cfg.BM, cfg.BN, cfg.BK, cfg.warp_m, cfg.warp_n, cfg.stages)]
+    rows, cols = tile_grid(cfg, M, N)
+    wgs = min(2, gemm_tc_occupancy(cfg, arch))
+    full, rest = divmod(rows * cols, arch.sm_nums * wgs)
+    t = 1.5 + full * (fixed + K // cfg.BK * (one if wgs == 1 else two))
+    if rest:
+        t += fixed + K // cfg.BK * (one if rest <= arch.sm_nums else two)
+    # between the orders of one tile: operand panels that an XCD's tiles fetch
+    per_xcd = min(rows * cols, arch.sm_nums * wgs) / getattr(arch, "num_xcd", 8)
+    band = min(cfg.raster or 8, per_xcd)
+    panels = band * cfg.BM + math.ceil(per_xcd / band) * cfg.BN
+    t *= 1.0 + 1e-5 * panels
+    return 2.0 * M * N * K / (arch.peak_mma_sync_flops * 1e3 * t)
 
 
 def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
@@ -169,9 +209,14 @@ def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
     - epilogue: C is written once; direct stores are 8-byte row segments, the
       staged epilogue writes 16-byte coalesced chunks
     """
+    from deca_amd.kernels.gemm_hip import tile_grid
+
+    if getattr(cfg, "edge", False):
+        return gemm_edge_score(cfg, arch, M, N, K)
     wgs = gemm_tc_occupancy(cfg, arch)
     slots = arch.sm_nums * wgs
-    grid = (M // cfg.BM) * (N // cfg.BN)
+    rows, cols = tile_grid(cfg, M, N)
+    grid = rows * cols
     wave_eff = _wave_efficiency(grid, slots)
     if getattr(cfg, "tail", False):
         # the partial last wave runs as quarter tiles: a quarter of the work each, at the
@@ -205,7 +250,7 @@ def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
         rows_x, cols_x = 8, max(1, per_xcd // 8)
     else:
         rows_x = min(cfg.raster, per_xcd)
-        cols_x = min(N // cfg.BN, math.ceil(per_xcd / rows_x))
+        cols_x = min(cols, math.ceil(per_xcd / rows_x))
     fabric_bpf = (rows_x * cfg.BM + cols_x * cfg.BN) / (per_xcd * cfg.BM * cfg.BN)
     t_fabric = fabric_bpf * cus / (getattr(arch, "mall_bw", arch.l2_bw) * 1e9)
     terms = sorted([t_mma, t_lds, t_l2, t_dram, t_fabric])

@@ -13,6 +13,14 @@
 //   DECA_EPI_LDS  1: stage C through LDS for 16-byte stores
 //   DECA_XCD      1: remap workgroup ids so that each of the 8 XCDs (private L2)
 //                 owns a contiguous slab of tiles
+//   DECA_EDGE     1: the tiles need not divide M and N: the last row and column of tiles
+//                 reach over the edge, with clamped loads and masked stores.  A shape whose
+//                 dimensions are multiples of 64 and of little else otherwise only gets
+//                 tiles of 64 rows or columns and grids of many uneven rounds: 1344 x
+//                 2816 x 5440 fp16 ran at 97 us with 462 tiles of 64 x 128 (53-61 us with
+//                 the best of them) and takes 42.6 us with 242 of 128 x 128, one per CU,
+//                 the last row of which is half empty.  Bound then: operand traffic, 32 KiB
+//                 per K-tile at 70 KB/us and CU (L2 hits and the fabric behind the L2)
 //   DECA_DIRECT   1: global -> LDS loads that bypass the VGPRs, ring of
 //                 DECA_STAGES (2..5) tiles; 0: loads staged through VGPRs one
 //                 tile ahead, ring of 1 or 2 tiles
@@ -49,6 +57,9 @@
 #endif
 #ifndef DECA_TAIL
 #define DECA_TAIL 0
+#endif
+#ifndef DECA_EDGE
+#define DECA_EDGE 0
 #endif
 
 #define M_ DECA_M
@@ -142,7 +153,8 @@ constexpr int LDS_BYTES = full_tile::LDS_BYTES > quarter_tile::LDS_BYTES ? full_
 #else
 constexpr int LDS_BYTES = full_tile::LDS_BYTES;
 #endif
-static_assert(DECA_RASTER == 0 || GM % (DECA_RASTER ? DECA_RASTER : 1) == 0,
+static_assert(!DECA_EDGE || DECA_TAIL == 0, "the tail is split over whole tiles");
+static_assert(DECA_RASTER == 0 || DECA_EDGE || GM % (DECA_RASTER ? DECA_RASTER : 1) == 0,
               "raster group must divide the workgroup rows");
 static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 
@@ -207,14 +219,18 @@ deca_main(const elem_t* __restrict__ A, const elem_t* __restrict__ B,
     // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a
     // contiguous range of tiles so that its L2 sees a compact set of A rows
     // and B columns.
-    static_assert(TILES % 8 == 0, "XCD remap needs a multiple of 8 workgroups");
-    lin = (lin & 7) * (TILES / 8) + (lin >> 3);
+    static_assert(DECA_EDGE || TILES % 8 == 0, "XCD remap needs a multiple of 8 workgroups");
+    // (the first TILES % 8 XCDs take one tile more)
+    lin = (lin & 7) * (TILES / 8) + min(lin & 7, TILES % 8) + (lin >> 3);
 #endif
   }
   {
     constexpr int GROUP = DECA_RASTER * GN;
-    bm = (lin / GROUP) * DECA_RASTER + (lin % GROUP) % DECA_RASTER;
-    bn = (lin % GROUP) / DECA_RASTER;
+    const int first = (lin / GROUP) * DECA_RASTER;
+    // (an odd last group of rows is shorter)
+    const int rows = GM % DECA_RASTER ? min(GM - first, DECA_RASTER) : DECA_RASTER;
+    bm = first + (lin % GROUP) % rows;
+    bn = (lin % GROUP) / rows;
   }
 #endif
 

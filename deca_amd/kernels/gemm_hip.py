@@ -75,6 +75,9 @@ class GemmConfig:
     # tile opens one group behind the barrier that frees its ring slot and runs into the
     # next K-tile (measured: +2 % at 4096^3, +6 % at 8192^3, +7.5 % at 16384^3 with 6).
     spread: int = 0
+    # the workgroup tiles need not divide M and N (nor their number be a multiple of 8): the
+    # last row and column of tiles reach over the edge of C
+    edge: bool = False
 
     @property
     def num_warps(self) -> int:
@@ -98,7 +101,13 @@ class GemmConfig:
             + (f",early={self.early}" if self.early else "")
             + (",agpr=1" if self.agpr else "")
             + (f",spread={self.spread}" if self.spread else "")
+            + (",edge=1" if self.edge else "")
         )
+
+
+def tile_grid(cfg: GemmConfig, M: int, N: int) -> tuple:
+    """Rows and columns of workgroup tiles."""
+    return -(-M // cfg.BM), -(-N // cfg.BN)
 
 
 # Groups behind a K-tile's barrier that pass before the first load of the spread window.
@@ -248,7 +257,13 @@ def check_config(cfg: GemmConfig, M: int, N: int, K: int, max_smem: int = MAX_LD
     assert cfg.warp_m % MFMA_M == 0 and cfg.warp_n % MFMA_M == 0
     assert cfg.BM % cfg.warp_m == 0 and cfg.BN % cfg.warp_n == 0
     assert cfg.BN >= 64
-    assert M % cfg.BM == 0 and N % cfg.BN == 0 and K % cfg.BK == 0
+    assert K % cfg.BK == 0
+    if cfg.edge:
+        # the loads of the last tiles are clamped by whole 16-byte chunks; the tail's quarter
+        # tiles have no edge
+        assert cfg.direct and not cfg.tail and N % 8 == 0
+    else:
+        assert M % cfg.BM == 0 and N % cfg.BN == 0
     assert WAVE <= cfg.threads <= 1024
     # Every lane issues the same number of 16-byte loads for each operand.
     assert (cfg.BM * cfg.BK // 8) % cfg.threads == 0
@@ -275,11 +290,12 @@ def check_config(cfg: GemmConfig, M: int, N: int, K: int, max_smem: int = MAX_LD
             q_head = spread_head_loads(q_loads, max(1, cfg.warp_m // 32), cfg.BK // 32, cfg.early, cfg.spread)
             assert (qs - 2) * q_loads + q_head <= 63
     if cfg.raster == 0:
-        full = (M // cfg.BM) * (N // cfg.BN) - (tail_tiles(cfg, M, N) if cfg.tail else 0)
-        assert cfg.xcd and (M // cfg.BM) % 8 == 0 and (N // cfg.BN) % 4 == 0 and full % 256 == 0
+        rows, cols = tile_grid(cfg, M, N)
+        full = rows * cols - (tail_tiles(cfg, M, N) if cfg.tail else 0)
+        assert cfg.xcd and rows % 8 == 0 and cols % 4 == 0 and full % 256 == 0
     else:
-        assert (M // cfg.BM) % cfg.raster == 0
-    if cfg.xcd:  # the remap permutes the full tiles
+        assert cfg.edge or (M // cfg.BM) % cfg.raster == 0
+    if cfg.xcd and not cfg.edge:  # the remap permutes the full tiles
         full = (M // cfg.BM) * (N // cfg.BN) - (tail_tiles(cfg, M, N) if cfg.tail else 0)
         assert full % 8 == 0
     if cfg.epi_smem:
@@ -313,7 +329,10 @@ def make_gemm_tc(M: int, N: int, K: int, cfg: GemmConfig, dtype: str = "float16"
     if cfg.spread:
         defines["DECA_DMA_SPREAD"] = cfg.spread
         defines["DECA_DMA_FIRST"] = SPREAD_FIRST
-    workgroups = (M // cfg.BM) * (N // cfg.BN)
+    if cfg.edge:
+        defines["DECA_EDGE"] = 1
+    rows, cols = tile_grid(cfg, M, N)
+    workgroups = rows * cols
     if cfg.tail:
         r = tail_tiles(cfg, M, N)
         defines["DECA_TAIL"] = r

@@ -156,8 +156,24 @@ GEMM_BF16_CASES = [
 ]
 
 
+# tiles that reach over the edge of C: one row or 8 columns in the last tile, one missing, both
+# edges at once, an edge in one dimension only, numbers of tiles that are no multiple of 8 or
+# of the tile order's rows, all three epilogues' stores (staged, direct), both tile forms
+GEMM_EDGE_CASES = [
+    (257, 264, 128, GemmConfig(256, 256, 64, 128, 64, 2, 2, True, mfma=16, early=4, agpr=True, spread=6, edge=True)),
+    (255, 504, 192, GemmConfig(128, 128, 64, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, edge=True)),
+    (320, 448, 320, GemmConfig(128, 256, 64, 64, 64, 3, 2, True, mfma=16, early=2, agpr=True, spread=3, edge=True)),
+    (64, 1088, 256, GemmConfig(256, 128, 64, 64, 64, 3, 1, True, mfma=16, early=2, spread=3, edge=True)),
+    (512, 712, 256, GemmConfig(128, 64, 64, 64, 32, 3, 1, False, mfma=16, early=2, agpr=True, edge=True)),
+    (1, 8, 192, GemmConfig(64, 128, 64, 64, 32, 3, 1, True, mfma=16, early=2, agpr=True, spread=3, edge=True)),
+    (833, 776, 320, GemmConfig(64, 64, 64, 32, 32, 5, 8, True, mfma=16, agpr=True, edge=True)),
+    (320, 200, 128, GemmConfig(128, 128, 32, 64, 64, 3, 2, False, edge=True)),
+    (960, 320, 128, GemmConfig(128, 64, 64, 64, 32, 2, 4, True, xcd=False, edge=True)),
+]
+
+
 def gemm_specs():
-    return ([make_gemm_tc(M, N, K, cfg) for M, N, K, cfg in GEMM_CASES + GEMM_FULL] +
+    return ([make_gemm_tc(M, N, K, cfg) for M, N, K, cfg in GEMM_CASES + GEMM_EDGE_CASES + GEMM_FULL] +
             [make_gemm_tc(M, N, K, cfg, "bfloat16") for M, N, K, cfg in GEMM_BF16_CASES])
 
 
