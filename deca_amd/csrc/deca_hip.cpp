@@ -133,6 +133,17 @@ int deca_launch(void* fn, unsigned gx, unsigned gy, unsigned gz, unsigned bx, un
                                   lds_bytes, static_cast<hipStream_t>(stream), params, nullptr));
 }
 
+int deca_launch_plan(const deca_plan* plan, void* stream, void* a, void* b, void* c, void* d) {
+  if (!plan || !plan->fn || plan->nargs > 4 ||
+      !geometry_ok(plan->grid[0], plan->grid[1], plan->grid[2], plan->block[0], plan->block[1],
+                   plan->block[2], plan->nargs))
+    return rc(hipErrorInvalidValue);
+  void* params[4] = {&a, &b, &c, &d};
+  return rc(hipModuleLaunchKernel(static_cast<hipFunction_t>(plan->fn), plan->grid[0], plan->grid[1],
+                                  plan->grid[2], plan->block[0], plan->block[1], plan->block[2],
+                                  plan->lds_bytes, static_cast<hipStream_t>(stream), params, nullptr));
+}
+
 int deca_launch_timed(void* fn, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned by,
                       unsigned bz, unsigned lds_bytes, void* stream, void* const* args,
                       unsigned nargs, unsigned nsets, unsigned iters, float* ms_total) {

@@ -107,6 +107,23 @@ int deca_launch(void* fn, unsigned gx, unsigned gy, unsigned gz,
                 unsigned bx, unsigned by, unsigned bz, unsigned lds_bytes,
                 void* stream, void* const* args, unsigned nargs);
 
+/* What does not change between the launches of a loaded kernel: its handle (valid
+ * until the module is unloaded) and geometry, laid out once by the caller. */
+typedef struct deca_plan {
+  void* fn;
+  unsigned grid[3];
+  unsigned block[3];
+  unsigned lds_bytes;
+  unsigned nargs;          /* device pointers the kernel takes: 1 to 4 */
+} deca_plan;
+
+/* deca_launch for kernels of up to four pointers, with everything that is the
+ * same on every call in `plan` and the pointers passed by value (the first
+ * plan->nargs of them count): a call from Python converts six integers instead
+ * of eleven and builds no array.  The plan is only read. */
+int deca_launch_plan(const deca_plan* plan, void* stream, void* a, void* b,
+                     void* c, void* d);
+
 /* Launches `fn` `iters` times back to back on `stream` between two events and
  * stores the elapsed milliseconds of the whole batch in `*ms_total`; blocks
  * until the batch has finished.  Launch i uses the argument set
