@@ -393,10 +393,10 @@ def solve_gemm_tc(arch, M: int, N: int, K: int, type_size: int = 2, count: int =
 
 def _edge_forms(arch, M: int, N: int, K: int):
     """GEMM configs whose workgroup tiles need not divide M and N (`edge`), for shapes that
-    are no multiple of 256 both ways: the eight-wave tile bodies measured on such shapes
-    (`cost_model.GEMM_STEP_TIMES`), in every tile order, down to half a tile per CU.  (A grid
-    of 242 tiles of 128 x 128 is 1.9x faster than 462 of 64 x 128, the best that divide
-    1344 x 2816.)"""
+    are no multiple of 256 both ways or have fewer tiles of 256 x 256 than there are CUs: the
+    tile bodies measured on such shapes (`cost_model.GEMM_STEP_TIMES`), in every tile order.  (A grid of 242 tiles of 128 x 128 is 1.25x faster than 462 of
+    64 x 128 and 2.3x faster than what was ranked first of those that divide 1344 x 2816; of 32
+    shapes measured both ways the form ranked first was never the slower one.)"""
     from dataclasses import replace
 
     from deca_amd.cost_model.CostModel import GEMM_STEP_TIMES
@@ -404,17 +404,22 @@ def _edge_forms(arch, M: int, N: int, K: int):
         GemmConfig, agpr_split_fits, check_config, default_spread, tile_grid,
     )
 
-    if (M % 256 == 0 and N % 256 == 0) or N % 8:
+    even = M % 256 == 0 and N % 256 == 0
+    if N % 8 or (even and M * N >= 256 * 256 * arch.sm_nums):
         return []
     results = []
-    for bm, bn, bk, wm, wn, st in GEMM_STEP_TIMES:
+    for bm, bn, bk, wm, wn, st, kg in GEMM_STEP_TIMES:
         if K % bk or K // bk < st:
             continue
         cfg = GemmConfig(BM=bm, BN=bn, BK=bk, warp_m=wm, warp_n=wn, stages=st, epi_smem=True,
-                         mfma=16, early=wm // 32 if wm >= 64 else 0, edge=True)
+                         mfma=16, early=wm // 32 if wm >= 64 else 0, edge=True, kgroups=kg)
         cfg = replace(cfg, agpr=agpr_split_fits(cfg), spread=default_spread(cfg))
         rows, cols = tile_grid(cfg, M, N)
-        if 2 * rows * cols < arch.sm_nums:
+        # A single round that leaves CUs idle: where smaller tiles come out even (multiples of
+        # 256) it loses from 30 % on, elsewhere it may still win at half (1664 x 640: 130 tiles
+        # of 64 x 128 against 260 of 64 x 64).  Wave groups pay while they are a CU's only
+        # waves (512 x 4096, two tiles per CU: the plain 64 x 128 tile is 10-20 % ahead).
+        if rows * cols < (0.7 if even else 0.5) * arch.sm_nums or (kg > 1 and rows * cols > arch.sm_nums):
             continue
         for ras in GEMM_RASTERS:
             if 0 < ras <= rows:

@@ -145,20 +145,21 @@ def gemm_mma_peak(cfg, arch) -> float:
 
 
 # Measured times of the eight-wave tile bodies (16x16x32 tiles, accumulators in AGPRs where
-# they fit, load window): (BM, BN, BK, warp_m, warp_n, stages) -> microseconds of
+# they fit, load window): (BM, BN, BK, warp_m, warp_n, stages, kgroups) -> microseconds of
 # (a workgroup's prologue and epilogue, one K-tile of a workgroup alone on its CU, one K-tile
 # of each of two on a CU).  Fitted to seven shapes that are multiples of 64 and of little else
 # (M 704 ... 4800, N 640 ... 7360, K 512 ... 5440); the times these give are within 10 % there.
 # What they show is the CU's load path and the fabric behind its L2 rather than the matrix pipe:
 # 32 KiB per 128 x 128 K-tile at 70 KB/us and CU.
 GEMM_STEP_TIMES = {
-    (256, 256, 64, 128, 64, 2): (6.0, 1.154, 2.308),
-    (256, 128, 64, 64, 64, 3): (2.6, 0.776, 1.552),
-    (128, 256, 64, 64, 64, 3): (2.7, 0.757, 1.514),
-    (128, 128, 64, 64, 32, 3): (1.3, 0.476, 0.952),
-    (128, 64, 64, 64, 32, 3): (1.0, 0.304, 0.594),
-    (64, 128, 64, 64, 32, 3): (1.0, 0.301, 0.597),
-    (64, 64, 64, 32, 32, 5): (1.0, 0.225, 0.390),
+    (256, 256, 64, 128, 64, 2, 1): (6.0, 1.154, 2.308),
+    (256, 128, 64, 64, 64, 3, 1): (2.6, 0.776, 1.552),
+    (128, 256, 64, 64, 64, 3, 1): (2.7, 0.757, 1.514),
+    (128, 128, 64, 64, 32, 3, 1): (1.3, 0.476, 0.952),
+    (128, 64, 64, 64, 32, 3, 1): (1.0, 0.304, 0.594),
+    (64, 128, 64, 64, 32, 3, 1): (1.0, 0.301, 0.597),
+    (64, 64, 64, 32, 32, 5, 1): (1.0, 0.225, 0.390),
+    (64, 64, 128, 64, 32, 3, 2): (1.0, 0.410, 0.820),
 }
 
 
@@ -167,7 +168,8 @@ def gemm_edge_score(cfg, arch, M: int, N: int, K: int) -> float:
     `GEMM_STEP_TIMES` gives it."""
     from deca_amd.kernels.gemm_hip import tile_grid
 
-    fixed, one, two = GEMM_STEP_TIMES[(cfg.BM, cfg.BN, cfg.BK, cfg.warp_m, cfg.warp_n, cfg.stages)]
+    fixed, one, two = GEMM_STEP_TIMES[(cfg.BM, cfg.BN, cfg.BK, cfg.warp_m, cfg.warp_n, cfg.stages,
+                                       cfg.kgroups)]
     rows, cols = tile_grid(cfg, M, N)
     wgs = min(2, gemm_tc_occupancy(cfg, arch))
     full, rest = divmod(rows * cols, arch.sm_nums * wgs)

@@ -21,6 +21,15 @@
 //                 the best of them) and takes 42.6 us with 242 of 128 x 128, one per CU,
 //                 the last row of which is half empty.  Bound then: operand traffic, 32 KiB
 //                 per K-tile at 70 KB/us and CU (L2 hits and the fabric behind the L2)
+//   DECA_KGROUPS  n > 1 (16x16x32 body): n groups of waves each hold all of the tile's
+//                 accumulators and take 1 / n of the k-steps of every K-tile; their sums
+//                 meet in LDS at the end (fp32).  For 64 x 64 tiles, of which a CU of a
+//                 256-workgroup grid has one: with K-tiles of 128 and two groups of 64 x 32
+//                 wave tiles there are half as many barriers and three quarters of the LDS
+//                 reads (compute side alone, four waves of 32 x 32 and K-tiles of 64: 547
+//                 clocks per K-tile for 128 of matrix work).  1024^3 fp16: 6.0 -> 4.8 us,
+//                 256 x 4096 x 4096 bf16: 16.9 -> 15.2 us; the loads alone (128 KiB in
+//                 flight, 1 MiB per CU from L2) take 15.5 us of the latter
 //   DECA_DIRECT   1: global -> LDS loads that bypass the VGPRs, ring of
 //                 DECA_STAGES (2..5) tiles; 0: loads staged through VGPRs one
 //                 tile ahead, ring of 1 or 2 tiles
@@ -60,6 +69,9 @@
 #endif
 #ifndef DECA_EDGE
 #define DECA_EDGE 0
+#endif
+#ifndef DECA_KGROUPS
+#define DECA_KGROUPS 1
 #endif
 
 #define M_ DECA_M
@@ -153,6 +165,7 @@ constexpr int LDS_BYTES = full_tile::LDS_BYTES > quarter_tile::LDS_BYTES ? full_
 #else
 constexpr int LDS_BYTES = full_tile::LDS_BYTES;
 #endif
+static_assert(DECA_KGROUPS == 1 || DECA_TAIL == 0, "the quarter tiles have one wave group");
 static_assert(!DECA_EDGE || DECA_TAIL == 0, "the tail is split over whole tiles");
 static_assert(DECA_RASTER == 0 || DECA_EDGE || GM % (DECA_RASTER ? DECA_RASTER : 1) == 0,
               "raster group must divide the workgroup rows");

@@ -78,10 +78,14 @@ class GemmConfig:
     # the workgroup tiles need not divide M and N (nor their number be a multiple of 8): the
     # last row and column of tiles reach over the edge of C
     edge: bool = False
+    # 16x16x32 body: groups of waves that share the k-steps of a K-tile, each with all of the
+    # tile's accumulators; the sums meet in LDS (fp32).  More waves per SIMD and fewer barriers
+    # (K-tiles of 128) for tiles too small to fill a CU's SIMDs
+    kgroups: int = 1
 
     @property
     def num_warps(self) -> int:
-        return (self.BM // self.warp_m) * (self.BN // self.warp_n)
+        return (self.BM // self.warp_m) * (self.BN // self.warp_n) * self.kgroups
 
     @property
     def threads(self) -> int:
@@ -102,6 +106,7 @@ class GemmConfig:
             + (",agpr=1" if self.agpr else "")
             + (f",spread={self.spread}" if self.spread else "")
             + (",edge=1" if self.edge else "")
+            + (f",kg={self.kgroups}" if self.kgroups != 1 else "")
         )
 
 
@@ -116,7 +121,7 @@ SPREAD_FIRST = 1
 
 def mfma_groups_per_ktile(cfg: GemmConfig) -> int:
     """MFMA groups (one row block against every column block) of a K-tile in the 16x16x32 body."""
-    return (cfg.BK // 32) * (cfg.warp_m // 16)
+    return cfg.BK // 32 // cfg.kgroups * (cfg.warp_m // 16)
 
 
 def spread_head_loads(loads: int, mt: int, ks: int, early: int, spread: int) -> int:
@@ -154,6 +159,8 @@ def pipeline_smem_bytes(cfg: GemmConfig) -> int:
 
 
 def epilogue_smem_bytes(cfg: GemmConfig) -> int:
+    if cfg.kgroups > 1:
+        return cfg.kgroups * cfg.BM * (cfg.BN + 4) * 4
     return cfg.BM * (cfg.BN + EPI_PAD) * 2 if cfg.epi_smem else 0
 
 
@@ -223,7 +230,8 @@ def accumulator_moves(cfg: GemmConfig) -> int:
     regs = (cfg.warp_m // 16) * (cfg.warp_n // 16) * 4
     if cfg.tail:
         regs += (cfg.warp_m // 32) * (cfg.warp_n // 32) * 4
-    return 2 * regs
+    # (the sums of wave groups go to LDS straight from the accumulation registers)
+    return regs if cfg.kgroups > 1 else 2 * regs
 
 
 def target_waves_per_simd(cfg: GemmConfig) -> int:
@@ -241,12 +249,15 @@ def check_config(cfg: GemmConfig, M: int, N: int, K: int, max_smem: int = MAX_LD
     assert cfg.stages in ((2, 3, 4, 5) if cfg.direct else (1, 2))
     assert K // cfg.BK >= cfg.stages
     assert smem_bytes(cfg) <= max_smem
-    assert cfg.BK in (32, 64)
+    assert cfg.BK in (32, 64) or (cfg.BK == 128 and cfg.mfma == 16)
+    assert cfg.kgroups in (1, 2, 4)
+    if cfg.kgroups > 1:
+        assert cfg.mfma == 16 and cfg.epi_smem and not cfg.tail and (cfg.BK // 32) % cfg.kgroups == 0
     assert cfg.mfma in (32, 16)
     if cfg.mfma == 16:
         # k-steps of 32; with one k-step per K-tile the main loop takes two tiles at a time
         assert cfg.direct
-        assert cfg.BK == 64 or (K // cfg.BK) % 2 == 0
+        assert cfg.BK // 32 // cfg.kgroups % 2 == 0 or (K // cfg.BK) % 2 == 0
         assert 0 <= cfg.early < cfg.warp_m // 16
         # 64 accumulator tiles of 16 x 16 per wave: hipcc fills all 256 accumulation and
         # all 256 vector registers and still spills 30-170 inside the loop (8x slower)
@@ -272,7 +283,7 @@ def check_config(cfg: GemmConfig, M: int, N: int, K: int, max_smem: int = MAX_LD
         # loads left in flight by the (stages - 2) youngest tiles -- and, with `spread`, the
         # head of the next one in the prologue -- fit the 6-bit counter
         loads = (cfg.BM * cfg.BK + cfg.BK * cfg.BN) // 8 // cfg.threads
-        head = spread_head_loads(loads, cfg.warp_m // 16, cfg.BK // 32, cfg.early, cfg.spread)
+        head = spread_head_loads(loads, cfg.warp_m // 16, cfg.BK // 32 // cfg.kgroups, cfg.early, cfg.spread)
         assert (cfg.stages - 2) * loads + head <= 63
     if cfg.tail:
         r = tail_tiles(cfg, M, N)
@@ -331,6 +342,8 @@ def make_gemm_tc(M: int, N: int, K: int, cfg: GemmConfig, dtype: str = "float16"
         defines["DECA_DMA_FIRST"] = SPREAD_FIRST
     if cfg.edge:
         defines["DECA_EDGE"] = 1
+    if cfg.kgroups > 1:
+        defines["DECA_KGROUPS"] = cfg.kgroups
     rows, cols = tile_grid(cfg, M, N)
     workgroups = rows * cols
     if cfg.tail:

@@ -169,6 +169,14 @@ GEMM_EDGE_CASES = [
     (833, 776, 320, GemmConfig(64, 64, 64, 32, 32, 5, 8, True, mfma=16, agpr=True, edge=True)),
     (320, 200, 128, GemmConfig(128, 128, 32, 64, 64, 3, 2, False, edge=True)),
     (960, 320, 128, GemmConfig(128, 64, 64, 64, 32, 2, 4, True, xcd=False, edge=True)),
+    # K-tiles of 128 and groups of waves that share their k-steps (two and four groups, an odd
+    # number of k-steps per group, the smallest number of K-tiles, with and without the edge)
+    (128, 192, 384, GemmConfig(64, 64, 128, 64, 32, 3, 2, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, xcd=False)),
+    (256, 256, 1152, GemmConfig(64, 64, 128, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
+    (100, 136, 512, GemmConfig(64, 64, 128, 64, 32, 4, 1, True, mfma=16, early=2, agpr=True, kgroups=4, edge=True)),
+    (256, 264, 256, GemmConfig(128, 128, 64, 64, 64, 3, 1, True, mfma=16, early=2, agpr=True, kgroups=2, edge=True)),
+    (192, 128, 512, GemmConfig(64, 64, 128, 32, 32, 4, 3, True, mfma=16, agpr=True, xcd=False)),
+    (128, 128, 256, GemmConfig(64, 64, 64, 32, 32, 3, 1, True, mfma=16, kgroups=2, xcd=False)),
 ]
 
 

@@ -1,5 +1,6 @@
-"""GPU parity of GEMM tiles that reach over the edge of C, by the checks of test_gemm_gpu.py,
-with rows behind C and the operands that nothing may write or need."""
+"""GPU parity of GEMM tiles that reach over the edge of C, and of K-tiles shared by groups of
+waves, by the checks of test_gemm_gpu.py, with rows behind C and the operands that nothing may
+write or need."""
 
 import pytest
 import torch
