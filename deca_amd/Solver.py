@@ -248,13 +248,23 @@ def solve_rowwise(
     reg_only = _rowwise_constraints(arch, op, M, N, type_size, force_reg=True)
     force_reg = N < twopass_min_n and _satisfiable(ROWWISE_DOMAINS, reg_only, backend)
     cons = reg_only if force_reg else _rowwise_constraints(arch, op, M, N, type_size, False)
-    return [
+    configs = [
         RowConfig(
             threads_per_row=tpr, rows_per_block=rpb, vec=vec,
             mode="twopass" if mode else "reg", unroll=unroll, hint=bool(hint),
         )
         for tpr, rpb, vec, mode, unroll, hint in _enumerate(ROWWISE_DOMAINS, cons, count, backend)
     ]
+    if N % 8 == 4 and configs:
+        # rows that are an odd multiple of 8 bytes: the forms of the next longer row that
+        # take 16-byte accesses, with half a vector at the end
+        longer = _rowwise_constraints(arch, op, M, N + 4, type_size, force_reg=True)
+        for tpr, rpb, vec, _, _, hint in _enumerate(ROWWISE_DOMAINS, longer, count, backend):
+            # (several rows a workgroup: from two workgroups per CU; 512 x 50004 loses 12 %)
+            if vec == 8 and tpr * vec <= N and (rpb == 1 or M // rpb >= 2 * arch.sm_nums):
+                configs.append(RowConfig(threads_per_row=tpr, rows_per_block=rpb, vec=8,
+                                         hint=bool(hint), half=True))
+    return configs[:count]
 
 
 # ---------------------------------------------------------------------------

@@ -67,6 +67,17 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     wgs = rowwise_occupancy(cfg, arch, op, N)
     chunks = num_chunks(cfg, N)
     depth = chunks if cfg.mode == "reg" else cfg.unroll
+    grid = M // cfg.rows_per_block
+    # every row resident at once: all loads are under way from the start, no round waits for
+    # another, and what is left to lose is the exchange between the waves of a row (RMSNorm
+    # 3001 x 5120: 10.6 us with one wave a row, 11.8 with two, 12.0 with four; eight take more
+    # than one round: 13.0; softmax 2000 x 8192: 11.4 with one, 12.7 with eight).  It takes
+    # about seven rows and 96 KiB per CU: below that (600 x 16384, 512 x 50004, 2048 x 4096)
+    # wider rows are 4-50 % ahead.
+    one_round = (cfg.mode == "reg" and grid <= arch.sm_nums * wgs and depth <= 16
+                 and M >= 7 * arch.sm_nums and M * N * type_size >= 96 * 1024 * arch.sm_nums)
+    if one_round:
+        wgs = max(1, math.ceil(grid / arch.sm_nums))
     in_flight = wgs * cfg.threads * depth * cfg.vec * type_size
     need = arch.dram_bw * 1e9 / arch.sm_nums * getattr(arch, "dram_latency_s", 2e-6)
     mem = min(1.0, in_flight / need)
@@ -74,7 +85,6 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     # (the loss levels off: 16 and 32 chunks per lane measure the same, 0.88 of the best)
     granularity = 1.0 / (1.0 + 0.012 * min(max(0, depth - 2), 11)) * (0.985 if depth == 1 else 1.0)
 
-    grid = M // cfg.rows_per_block
     wave_eff = _wave_efficiency(grid, arch.sm_nums * wgs)
     drain = 1.0 / (1.0 + 0.10 * max(0.0, cfg.threads / 256 - 2.0))
     rows = 1.0 / (1.0 + 0.015 * abs(math.log2(cfg.rows_per_block) - 1.0))
@@ -91,6 +101,9 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     reduce = 1.0 / (1.0 + 0.005 * math.log2(waves_per_row))
     if cfg.threads_per_row < arch.warp_size:
         reduce *= 0.97
+    if one_round:
+        wave_eff = granularity = 1.0
+        reduce *= 1.0 / (1.0 + 0.05 * math.log2(waves_per_row))
 
     tail = N / (chunks * cfg.threads_per_row * cfg.vec) if cfg.mode == "reg" else 1.0
     lanes = 1.0 if cfg.vec * type_size >= 16 else 0.985
@@ -371,7 +384,8 @@ def fa_split_score(cfg, arch, shape, causal: bool = False) -> float:
         mean = fixed + (S_kv / 2 + cfg.Br / 2) / (cfg.Bc * cfg.num_warps) * step
         t = max(longest, rounds * mean)
     else:
-        t = math.ceil(rounds) * longest
+        # (further rounds were 20 % longer than this at three: B4 H32 S_q 192 S_kv 1600 D 128)
+        t = math.ceil(rounds) * longest * (1.2 if rounds > 1 else 1.0)
     flops = 4.0 * B * H * S_q * S_kv * D * (0.5 if causal else 1.0)
     return flops / (arch.peak_mma_sync_flops * 1e9) / ((t - launch) * (0.8 if causal else 0.95))
 

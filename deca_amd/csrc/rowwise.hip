@@ -16,6 +16,12 @@
 //   DECA_HINT    1: non-temporal loads of read-once data and non-temporal stores
 //   DECA_LEAN    1 (reg mode): nothing but the packed row stays in registers between
 //                the reduction and the stores -- the fp32 values are computed again
+//   DECA_HALF    1 (reg mode, VEC = 8): N is an odd multiple of 4.  Rows then start on 8-byte
+//                boundaries only; the accesses are 16 bytes all the same (the hardware asks
+//                for 4-byte alignment) but for the last half vector of a row.  RMSNorm fp16
+//                3001 x 5124: 14.3 us with 8-byte accesses and 128 lanes a row, 11.4 us with
+//                these and a wave a row (3001 x 5120, whose rows are aligned: 10.6); softmax
+//                bf16 777 x 65532: 52.0 and 45.9 us
 //   DECA_EPS     RMSNorm epsilon
 //
 // Lane t of a row owns the VEC-element chunks (c * TPR + t) * VEC, so one wave
@@ -44,7 +50,11 @@
 #define RED_LANES (TPR < 64 ? TPR : 64)
 #define NW (TPR / 64 > 0 ? TPR / 64 : 1)
 
-static_assert(DECA_N % VEC == 0, "N must be a multiple of the vector width");
+#ifndef DECA_HALF
+#define DECA_HALF 0
+#endif
+static_assert(DECA_HALF ? (VEC == 8 && DECA_N % 8 == 4 && DECA_MODE == 0) : DECA_N % VEC == 0,
+              "N must be a multiple of the vector width, or of half of it (DECA_HALF)");
 static_assert(DECA_M % RPB == 0, "M must be a multiple of rows_per_block");
 static_assert(NT % 64 == 0 && NT <= 1024, "workgroup must be whole waves");
 static_assert(VEC == 8 || VEC == 4 || VEC == 2, "vec");
@@ -55,6 +65,12 @@ typedef __bf16 elem_t;
 typedef _Float16 elem_t;
 #endif
 typedef elem_t vec_t __attribute__((ext_vector_type(VEC)));
+#if DECA_HALF
+typedef elem_t half_t __attribute__((ext_vector_type(4)));
+typedef vec_t mem_t __attribute__((aligned(8)));  // a vector as it lies in memory
+#else
+typedef vec_t mem_t;
+#endif
 
 #ifndef DECA_LEAN
 #define DECA_LEAN 0
@@ -129,18 +145,21 @@ __device__ __forceinline__ float row_reduce(float v, Op op, float* red, int row_
 // ---------------------------------------------------------------------------
 // memory helpers
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ vec_t load_vec(const elem_t* p, bool once) {
+// (ONCE is a template parameter: as an argument, the two loads are merged before it is known
+// and the non-temporal hint is lost)
+template <bool ONCE>
+__device__ __forceinline__ vec_t load_vec(const elem_t* p) {
 #if DECA_HINT
-  if (once) return __builtin_nontemporal_load(reinterpret_cast<const vec_t*>(p));
+  if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const mem_t*>(p));
 #endif
-  return *reinterpret_cast<const vec_t*>(p);
+  return *reinterpret_cast<const mem_t*>(p);
 }
 
 __device__ __forceinline__ void store_vec(elem_t* p, vec_t v) {
 #if DECA_HINT
-  __builtin_nontemporal_store(v, reinterpret_cast<vec_t*>(p));
+  __builtin_nontemporal_store(v, reinterpret_cast<mem_t*>(p));
 #else
-  *reinterpret_cast<vec_t*>(p) = v;
+  *reinterpret_cast<mem_t*>(p) = v;
 #endif
 }
 
@@ -175,22 +194,44 @@ deca_main(const elem_t* __restrict__ x,
   auto col = [&](int c) { return (c * TPR + t) * VEC; };
   // Chunks >= C_FULL are out of the row for the upper lanes.
   auto in_row = [&](int c) { return c < C_FULL || col(c) < DECA_N; };
+#if DECA_HALF
+  // The last vector of a row: its upper half is beyond the end.
+  auto whole = [&](int c) { return c < C_FULL || col(c) + VEC <= DECA_N; };
+  auto elem_ok = [&](int c, int i) { return i < 4 ? in_row(c) : whole(c); };
+  auto load_half = [&](const elem_t* base, int c) {
+    const half_t h = *reinterpret_cast<const half_t*>(base + col(c));
+    const half_t none = {};
+    return __builtin_shufflevector(h, none, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  auto load_x = [&](int c) { return whole(c) ? load_vec<true>(xr + col(c)) : load_half(xr, c); };
+  auto load_w = [&](const elem_t* w, int c) { return whole(c) ? load_vec<false>(w + col(c)) : load_half(w, c); };
+  auto store_row = [&](int c, vec_t v) {
+    if (whole(c))
+      store_vec(yr + col(c), v);
+    else
+      *reinterpret_cast<half_t*>(yr + col(c)) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+  };
+#else
+  auto elem_ok = [&](int c, int) { return in_row(c); };
+  auto load_x = [&](int c) { return load_vec<true>(xr + col(c)); };
+  auto load_w = [&](const elem_t* w, int c) { return load_vec<false>(w + col(c)); };
+  auto store_row = [&](int c, vec_t v) { store_vec(yr + col(c), v); };
+#endif
 
 #if DECA_MODE == 0
   // ------------------------------ reg mode ------------------------------
   vec_t xh[NCHUNK];
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
-    if (in_row(c)) xh[c] = load_vec(xr + col(c), true);
+    if (in_row(c)) xh[c] = load_x(c);
   }
 
 #if DECA_OP == 0
   float m = NEG_INF;
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
-    const bool ok = in_row(c);
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) m = fmaxf(m, ok ? static_cast<float>(xh[c][i]) : NEG_INF);
+    for (int i = 0; i < VEC; ++i) m = fmaxf(m, elem_ok(c, i) ? static_cast<float>(xh[c][i]) : NEG_INF);
   }
   const float m2 = row_reduce(m, MaxOp(), red0, rb, wr, lane) * LOG2E;
 #if DECA_LEAN
@@ -201,10 +242,9 @@ deca_main(const elem_t* __restrict__ x,
   float s = 0.0f;
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
-    const bool ok = in_row(c);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
-      const float v = ok ? static_cast<float>(xh[c][i]) : NEG_INF;
+      const float v = elem_ok(c, i) ? static_cast<float>(xh[c][i]) : NEG_INF;
       s += fast_exp2(v * LOG2E - m2);
     }
   }
@@ -223,17 +263,16 @@ deca_main(const elem_t* __restrict__ x,
 #pragma unroll
       for (int i = 0; i < VEC; ++i)
         o[i] = static_cast<elem_t>(fast_exp2(static_cast<float>(xh[c][i]) * LOG2E - m2) * inv);
-      store_vec(yr + col(c), o);
+      store_row(c, o);
     }
   }
 #else
   float ss = 0.0f;
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
-    const bool ok = in_row(c);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
-      const float v = ok ? static_cast<float>(xh[c][i]) : 0.0f;
+      const float v = elem_ok(c, i) ? static_cast<float>(xh[c][i]) : 0.0f;
       ss += v * v;
     }
   }
@@ -247,14 +286,14 @@ deca_main(const elem_t* __restrict__ x,
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
     if (in_row(c)) {
-      const vec_t wv = *reinterpret_cast<const vec_t*>(w + col(c));
+      const vec_t wv = load_w(w, c);
       vec_t o;
 #pragma unroll
       for (int i = 0; i < VEC; ++i) {
         const float normed = static_cast<float>(static_cast<elem_t>(static_cast<float>(xh[c][i]) * r));
         o[i] = static_cast<elem_t>(normed * static_cast<float>(wv[i]));
       }
-      store_vec(yr + col(c), o);
+      store_row(c, o);
     }
   }
 #endif
@@ -304,7 +343,7 @@ deca_main(const elem_t* __restrict__ x,
     bool ok[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      v[u] = load_vec(xr + col(g * U + u), false);
+      v[u] = load_vec<false>(xr + col(g * U + u));
       ok[u] = true;
     }
     online(v, ok, U);
@@ -314,7 +353,7 @@ deca_main(const elem_t* __restrict__ x,
     vec_t v[1];
     bool ok[1];
     ok[0] = in_row(c);
-    if (ok[0]) v[0] = load_vec(xr + col(c), false);
+    if (ok[0]) v[0] = load_vec<false>(xr + col(c));
     online(v, ok, 1);
   }
 
@@ -348,13 +387,13 @@ deca_main(const elem_t* __restrict__ x,
   for (int g = 0; g < N_LOOP; ++g) {
     vec_t v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = load_vec(xr + col(g * U + u), true);
+    for (int u = 0; u < U; ++u) v[u] = load_vec<true>(xr + col(g * U + u));
 #pragma unroll
     for (int u = 0; u < U; ++u) emit(g * U + u, v[u]);
   }
 #pragma unroll
   for (int c = N_LOOP * U; c < NCHUNK; ++c) {
-    if (in_row(c)) emit(c, load_vec(xr + col(c), true));
+    if (in_row(c)) emit(c, load_vec<true>(xr + col(c)));
   }
 #endif
 }

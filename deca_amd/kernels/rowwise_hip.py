@@ -51,6 +51,9 @@ class RowConfig:
     mode: str = "reg"
     unroll: int = 1  # chunks loaded back to back per twopass iteration
     hint: bool = False  # non-temporal loads of read-once data and non-temporal stores
+    # rows whose length is an odd multiple of 4 in 16-byte accesses (vec = 8, reg mode), the
+    # last one of a row a half
+    half: bool = False
 
     @property
     def threads(self) -> int:
@@ -62,7 +65,7 @@ class RowConfig:
     def __str__(self):
         s = f"tpr={self.threads_per_row},rpb={self.rows_per_block},vec={self.vec},mode={self.mode}"
         s += f",unroll={self.unroll}" if self.mode == "twopass" else ""
-        return s + (",hint=1" if self.hint else "")
+        return s + (",hint=1" if self.hint else "") + (",half=1" if self.half else "")
 
 
 def num_chunks(cfg: RowConfig, N: int) -> int:
@@ -115,7 +118,11 @@ def regs_per_thread(cfg: RowConfig, N: int, op: str) -> int:
 
 def check_config(cfg: RowConfig, op: str, M: int, N: int, dtype: str) -> None:
     assert op in OPS and dtype in DTYPES and cfg.mode in MODES
-    assert cfg.vec in (2, 4, 8) and N % cfg.vec == 0
+    assert cfg.vec in (2, 4, 8)
+    if cfg.half:
+        assert cfg.vec == 8 and cfg.mode == "reg" and N % 8 == 4
+    else:
+        assert N % cfg.vec == 0
     assert not cfg.hint or cfg.vec in (4, 8), "cache hints need 8- or 16-byte accesses"
     assert cfg.threads_per_row in TPR_CHOICES
     assert cfg.threads % WAVE == 0 and cfg.threads <= MAX_THREADS
@@ -154,6 +161,8 @@ def make_rowwise(
     }
     if use_lean(cfg, N, op):
         defines["DECA_LEAN"] = 1
+    if cfg.half:
+        defines["DECA_HALF"] = 1
     return make_spec(
         TEMPLATE, defines, grid=(M // cfg.rows_per_block, 1, 1), block=(cfg.threads, 1, 1),
         nargs=3 if op == "rmsnorm" else 2, options=FAST_MATH_OPTIONS,

@@ -95,7 +95,8 @@ def parse_config(operator: str, text: str):
     elif operator in ("softmax", "rmsnorm"):
         fields.update(threads_per_row=int(pairs.pop("tpr")), rows_per_block=int(pairs.pop("rpb")),
                       vec=int(pairs.pop("vec")), mode=pairs.pop("mode"),
-                      unroll=int(pairs.pop("unroll", 1)), hint=bool(int(pairs.pop("hint", 0))))
+                      unroll=int(pairs.pop("unroll", 1)), hint=bool(int(pairs.pop("hint", 0))),
+                      half=bool(int(pairs.pop("half", 0))))
     else:
         fields.update(Br=int(pairs.pop("Br")), Bc=int(pairs.pop("Bc")),
                       num_warps=int(pairs.pop("warps")), stages=int(pairs.pop("stages")),

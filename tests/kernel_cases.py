@@ -46,6 +46,16 @@ ROWWISE_CASES = [
     ("rmsnorm", 512, 1024, "float16", RowConfig(32, 2, 8)),
     ("rmsnorm", 256, 4096, "bfloat16", RowConfig(64, 4, 8, "twopass", 2)),
     ("rmsnorm", 64, 32000, "float16", RowConfig(512, 2, 8, "twopass", 4, True)),
+    # 16-byte accesses on rows that are an odd multiple of 8 bytes, the last one a half: alone
+    # in its chunk, the last of a chunk, the first lane's, in the only chunk, with an odd row
+    # count (every other row starts off a 16-byte boundary), plain, hinted and lean
+    ("rmsnorm", 67, 5124, "float16", RowConfig(64, 1, 8, hint=True, half=True)),
+    ("softmax", 33, 1020, "float16", RowConfig(64, 1, 8, half=True)),
+    ("softmax", 64, 1028, "bfloat16", RowConfig(16, 4, 8, hint=True, half=True)),
+    ("rmsnorm", 30, 516, "bfloat16", RowConfig(64, 2, 8, hint=True, half=True)),
+    ("softmax", 12, 132, "float16", RowConfig(16, 4, 8, half=True)),
+    ("softmax", 9, 128252, "bfloat16", RowConfig(1024, 1, 8, hint=True, half=True)),
+    ("rmsnorm", 7, 128260, "float16", RowConfig(512, 1, 8, half=True)),
 ]
 
 # Full-size benchmark shapes (property checks + a sampled comparison).
