@@ -1,0 +1,28 @@
+"""Host test of the rankings on shapes where a rule once put the slower of two measured
+configurations first.  Times are microseconds per launch on an MI355X, launches back to back
+over buffers larger than the caches, both configurations in turn in one process."""
+
+import pytest
+
+from deca_amd import Solver
+from deca_amd.arch import MI355X
+from deca_amd.cost_model import CostModel as cm
+
+ARCH = MI355X()
+
+# (operator, M, N, the slower configuration, its time, a time another one of the solver's takes)
+ROWWISE = [
+    # two vectors a lane, the second part empty, and half a vector at the end of the row
+    ("softmax", 2713, 4116, "tpr=512,rpb=1,vec=8,mode=reg,hint=1,half=1", 11.7, 10.4),
+    ("softmax", 1449, 2748, "tpr=256,rpb=1,vec=8,mode=reg,hint=1,half=1", 5.4, 4.6),
+    ("softmax", 6309, 564, "tpr=64,rpb=1,vec=8,mode=reg,hint=1,half=1", 5.4, 4.9),
+    ("rmsnorm", 20359, 1044, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 21.3, 18.3),
+    ("rmsnorm", 611, 4820, "tpr=512,rpb=1,vec=8,mode=reg,hint=1,half=1", 4.5, 4.2),
+]
+
+
+@pytest.mark.parametrize("op,M,N,slower,slower_us,us", ROWWISE, ids=lambda v: str(v))
+def test_rowwise_first_rank_is_not_the_slower_form(op, M, N, slower, slower_us, us):
+    assert us < slower_us
+    first = cm.rank_rowwise_configs(Solver.solve_rowwise(ARCH, op, M, N), ARCH, op, M, N)[0]
+    assert str(first) != slower
