@@ -68,14 +68,18 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     chunks = num_chunks(cfg, N)
     depth = chunks if cfg.mode == "reg" else cfg.unroll
     grid = M // cfg.rows_per_block
-    # every row resident at once: all loads are under way from the start, no round waits for
-    # another, and what is left to lose is the exchange between the waves of a row (RMSNorm
-    # 3001 x 5120: 10.6 us with one wave a row, 11.8 with two, 12.0 with four; eight take more
-    # than one round: 13.0; softmax 2000 x 8192: 11.4 with one, 12.7 with eight).  It takes
-    # about seven rows and 96 KiB per CU: below that (600 x 16384, 512 x 50004, 2048 x 4096)
-    # wider rows are 4-50 % ahead.
-    one_round = (cfg.mode == "reg" and grid <= arch.sm_nums * wgs and depth <= 16
-                 and M >= 7 * arch.sm_nums and M * N * type_size >= 96 * 1024 * arch.sm_nums)
+    # One wave a row with every row resident at once: all loads are under way from the start, no
+    # round waits for another and no waves meet.  Measured against the choice without this term
+    # (60 shapes): RMSNorm 1.02-1.26x from 7 to 16 rows and 96 to 144 KiB per CU (3977 x 4992
+    # at 151 KiB still, nothing from 17 rows on: 5086 x 3464 0.96x); softmax, whose wave has
+    # twice the arithmetic per row to do alone, 1.02-1.26x up to 128 KiB and 0.95-1.02x beyond.
+    # Below 7 rows or 96 KiB (600 x 16384, 512 x 50004, 2048 x 4096) wider rows are 4-50 % ahead.
+    rows_per_cu = M / arch.sm_nums
+    kib_per_cu = rows_per_cu * N * type_size / 1024
+    one_round = (cfg.mode == "reg" and cfg.threads_per_row == arch.warp_size
+                 and cfg.rows_per_block == 1 and cfg.vec * type_size >= 16 and depth <= 16
+                 and grid <= arch.sm_nums * wgs and 7 <= rows_per_cu <= 16
+                 and 96 <= kib_per_cu <= (128 if op == "softmax" else 144))
     if one_round:
         wgs = max(1, math.ceil(grid / arch.sm_nums))
     in_flight = wgs * cfg.threads * depth * cfg.vec * type_size
@@ -103,7 +107,6 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
         reduce *= 0.97
     if one_round:
         wave_eff = granularity = 1.0
-        reduce *= 1.0 / (1.0 + 0.05 * math.log2(waves_per_row))
 
     tail = N / (chunks * cfg.threads_per_row * cfg.vec) if cfg.mode == "reg" else 1.0
     lanes = 1.0 if cfg.vec * type_size >= 16 else 0.985

@@ -18,6 +18,13 @@ ROWWISE = [
     ("softmax", 6309, 564, "tpr=64,rpb=1,vec=8,mode=reg,hint=1,half=1", 5.4, 4.9),
     ("rmsnorm", 20359, 1044, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 21.3, 18.3),
     ("rmsnorm", 611, 4820, "tpr=512,rpb=1,vec=8,mode=reg,hint=1,half=1", 4.5, 4.2),
+    # rows all resident at once: several rows a workgroup, fewer lanes than a wave or 8-byte
+    # accesses have nothing of what one wave a row gains there, nor has it with long softmax rows
+    ("softmax", 7338, 3000, "tpr=32,rpb=2,vec=8,mode=reg,hint=1", 18.2, 17.0),
+    ("softmax", 2718, 7408, "tpr=64,rpb=2,vec=8,mode=reg,hint=1", 17.1, 15.8),
+    ("softmax", 11580, 1648, "tpr=16,rpb=4,vec=8,mode=reg,hint=1", 17.0, 14.6),
+    ("rmsnorm", 4300, 3328, "tpr=64,rpb=2,vec=4,mode=reg,hint=1", 13.1, 10.6),
+    ("rmsnorm", 5950, 3448, "tpr=32,rpb=2,vec=8,mode=reg,hint=1", 17.7, 16.2),
 ]
 
 
