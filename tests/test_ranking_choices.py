@@ -33,3 +33,36 @@ def test_rowwise_first_rank_is_not_the_slower_form(op, M, N, slower, slower_us, 
     assert us < slower_us
     first = cm.rank_rowwise_configs(Solver.solve_rowwise(ARCH, op, M, N), ARCH, op, M, N)[0]
     assert str(first) != slower
+
+
+# (B, H, S_q, S_kv, D, causal, the slower configuration, its time, that of the plain form)
+ATTENTION = [
+    # few keys, more than two rows of 32 queries per CU: the plain forms fill the SIMDs too
+    (3, 16, 384, 384, 64, False, "Br=32,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 8.2, 7.1),
+    (5, 16, 384, 384, 64, False, "Br=64,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 10.5, 9.1),
+    (8, 8, 256, 256, 64, False, "Br=64,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 6.7, 5.9),
+    (6, 16, 384, 384, 64, True, "Br=64,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 11.0, 9.6),
+    (6, 8, 768, 768, 128, True, "Br=32,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 25.6, 21.9),
+]
+
+
+@pytest.mark.parametrize("B,H,S_q,S_kv,D,causal,slower,slower_us,us", ATTENTION, ids=lambda v: str(v))
+def test_attention_first_rank_is_not_the_slower_form(B, H, S_q, S_kv, D, causal, slower, slower_us, us):
+    assert us < slower_us
+    shape = (B, H, S_q, S_kv, D)
+    first = cm.rank_fa_configs(Solver.solve_flash_attn(ARCH, *shape), ARCH, shape, causal)[0]
+    assert str(first) != slower
+
+
+# (B, H, S_q, S_kv, D, causal): shapes on which a key-split form was measured 1.1 ... 3.7x ahead
+# of the plain form ranked first
+KEY_SPLIT = [
+    (1, 16, 512, 512, 64, True), (1, 16, 512, 8192, 128, False), (4, 8, 320, 384, 64, False),
+    (1, 8, 1216, 12096, 128, False), (2, 16, 768, 768, 64, True), (3, 16, 704, 704, 128, True),
+]
+
+
+@pytest.mark.parametrize("B,H,S_q,S_kv,D,causal", KEY_SPLIT)
+def test_attention_first_rank_is_the_key_split_where_it_is_ahead(B, H, S_q, S_kv, D, causal):
+    shape = (B, H, S_q, S_kv, D)
+    assert cm.rank_fa_configs(Solver.solve_flash_attn(ARCH, *shape), ARCH, shape, causal)[0].kv_split
