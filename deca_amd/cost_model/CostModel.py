@@ -179,13 +179,16 @@ GEMM_STEP_TIMES = {
 }
 
 
-def gemm_edge_score(cfg, arch, M: int, N: int, K: int) -> float:
-    """Score of an `edge` config: useful share of the matrix peak in the time that
-    `GEMM_STEP_TIMES` gives it."""
+def gemm_edge_score(cfg, arch, M: int, N: int, K: int) -> float | None:
+    """Score of a config by the step times of its tile body: useful share of the matrix peak in
+    the time that `GEMM_STEP_TIMES` gives it.  None for a body without an entry."""
     from deca_amd.kernels.gemm_hip import tile_grid
 
-    fixed, one, two = GEMM_STEP_TIMES[(cfg.BM, cfg.BN, cfg.BK, cfg.warp_m, cfg.warp_n, cfg.stages,
-                                       cfg.kgroups)]
+    times = GEMM_STEP_TIMES.get((cfg.BM, cfg.BN, cfg.BK, cfg.warp_m, cfg.warp_n, cfg.stages,
+                                 cfg.kgroups))
+    if times is None or cfg.mfma != 16:
+        return None
+    fixed, one, two = times
     rows, cols = tile_grid(cfg, M, N)
     wgs = min(2, gemm_tc_occupancy(cfg, arch))
     full, rest = divmod(rows * cols, arch.sm_nums * wgs)
@@ -230,7 +233,9 @@ def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
     from deca_amd.kernels.gemm_hip import tile_grid
 
     if getattr(cfg, "edge", False):
-        return gemm_edge_score(cfg, arch, M, N, K)
+        by_steps = gemm_edge_score(cfg, arch, M, N, K)
+        if by_steps is not None:
+            return by_steps
     wgs = gemm_tc_occupancy(cfg, arch)
     slots = arch.sm_nums * wgs
     rows, cols = tile_grid(cfg, M, N)
@@ -315,7 +320,9 @@ def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
             loads = (cfg.BM * cfg.BK + cfg.BK * cfg.BN) // 8 // cfg.threads
             form += 0.005 * loads
 
-    return form * wave_eff * hiding * pipe * sync_eff * staged / ((t_flop + t_epi) / t_mma)
+    # (tiles that reach over the edge of C compute more than the shape needs)
+    useful = M * N / (grid * cfg.BM * cfg.BN)
+    return useful * form * wave_eff * hiding * pipe * sync_eff * staged / ((t_flop + t_epi) / t_mma)
 
 
 def rank_gemm_configs(configs, arch, M: int, N: int, K: int, top_n: int | None = None,

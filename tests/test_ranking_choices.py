@@ -7,6 +7,7 @@ import pytest
 from deca_amd import Solver
 from deca_amd.arch import MI355X
 from deca_amd.cost_model import CostModel as cm
+from kernel_cases import GEMM_EDGE_CASES
 
 ARCH = MI355X()
 
@@ -66,3 +67,21 @@ KEY_SPLIT = [
 def test_attention_first_rank_is_the_key_split_where_it_is_ahead(B, H, S_q, S_kv, D, causal):
     shape = (B, H, S_q, S_kv, D)
     assert cm.rank_fa_configs(Solver.solve_flash_attn(ARCH, *shape), ARCH, shape, causal)[0].kv_split
+
+
+@pytest.mark.parametrize("M,N,K,cfg", GEMM_EDGE_CASES, ids=lambda v: str(v))
+def test_every_valid_edge_form_can_be_ranked(M, N, K, cfg):
+    """Also a tile body without measured step times."""
+    assert cm.rank_gemm_configs([cfg], ARCH, M, N, K) == [cfg]
+    assert 0.0 < cm.gemm_tc_score(cfg, ARCH, M, N, K) < 1.0
+
+
+def test_edge_score_counts_useful_work_only():
+    from dataclasses import replace
+
+    from deca_amd.kernels.gemm_hip import GemmConfig
+
+    # a body without step times: half of the last row of tiles is outside of C
+    cfg = GemmConfig(128, 128, 32, 64, 64, 3, 2, False, edge=True)
+    full, cut = (cm.gemm_tc_score(cfg, ARCH, M, 2048, 512) for M in (2048, 1984))
+    assert cut < full == cm.gemm_tc_score(replace(cfg, edge=False), ARCH, 2048, 2048, 512)
