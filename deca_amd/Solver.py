@@ -399,25 +399,28 @@ def solve_gemm_tc(arch, M: int, N: int, K: int, type_size: int = 2, count: int =
                         continue
                 results.append(cand)
     if results:
-        results += _edge_forms(arch, M, N, K)
+        # (where a tile divides C the `edge` form is the plain one's code once more)
+        plain = set(results)
+        results += [c for c in _edge_forms(arch, M, N, K) if replace(c, edge=False) not in plain]
     return results[:count]
 
 
 def _edge_forms(arch, M: int, N: int, K: int):
     """GEMM configs whose workgroup tiles need not divide M and N (`edge`), for shapes that
     are no multiple of 256 both ways or have fewer tiles of 256 x 256 than there are CUs: the
-    tile bodies measured on such shapes (`cost_model.GEMM_STEP_TIMES`), in every tile order.  (A grid of 242 tiles of 128 x 128 is 1.25x faster than 462 of
-    64 x 128 and 2.3x faster than what was ranked first of those that divide 1344 x 2816; of 32
-    shapes measured both ways the form ranked first was never the slower one.)"""
+    tile bodies measured on such shapes (`cost_model.GEMM_STEP_TIMES`), in every tile order.
+    (A grid of 242 tiles of 128 x 128 is 1.25x faster than 462 of 64 x 128 and 2.3x faster than
+    what was ranked first of those that divide 1344 x 2816.  Of 175 shapes measured both ways
+    the form ranked first was the slower one on 7, by 2 to 10 %.)"""
     from dataclasses import replace
 
-    from deca_amd.cost_model.CostModel import GEMM_STEP_TIMES
+    from deca_amd.cost_model.CostModel import GEMM_STEP_TIMES, gemm_step_times_apply
     from deca_amd.kernels.gemm_hip import (
         GemmConfig, agpr_split_fits, check_config, default_spread, tile_grid,
     )
 
     even = M % 256 == 0 and N % 256 == 0
-    if N % 8 or (even and M * N >= 256 * 256 * arch.sm_nums):
+    if N % 8 or not gemm_step_times_apply(arch, M, N):
         return []
     results = []
     for bm, bn, bk, wm, wn, st, kg in GEMM_STEP_TIMES:

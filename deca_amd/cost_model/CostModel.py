@@ -11,6 +11,7 @@ the winner.
 from __future__ import annotations
 
 import math
+from dataclasses import replace
 
 from deca_amd.driver.driver import cu_occupancy
 
@@ -203,9 +204,48 @@ def gemm_edge_score(cfg, arch, M: int, N: int, K: int) -> float | None:
     return 2.0 * M * N * K / (arch.peak_mma_sync_flops * 1e3 * t)
 
 
-def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
+def gemm_measured_form(cfg):
+    """The config of `cfg`'s tile body and order that `GEMM_STEP_TIMES` was measured with, None
+    for a body without an entry."""
+    from deca_amd.kernels.gemm_hip import agpr_split_fits, default_spread
+
+    if getattr(cfg, "mfma", 32) != 16 or not cfg.direct:
+        return None
+    for bm, bn, bk, wm, wn, stages, kgroups in GEMM_STEP_TIMES:
+        if (bm, bn, bk, wm, wn, kgroups) == (cfg.BM, cfg.BN, cfg.BK, cfg.warp_m, cfg.warp_n,
+                                             cfg.kgroups):
+            twin = replace(cfg, stages=stages, tail=False, epi_smem=True, xcd=True, edge=True,
+                           early=wm // 32 if wm >= 64 else 0, agpr=False, spread=0)
+            return replace(twin, agpr=agpr_split_fits(twin), spread=default_spread(twin))
+    return None
+
+
+def gemm_form_factor(cfg) -> float:
+    """What the form of a tile's loop is worth beside the terms of `gemm_general_score`."""
+    # 16x16x32 tiles: measured ahead of the 32x32x16 twin where the grid is a single wave of
+    # workgroups or leaves a partial one (2048^3 +7 %, 4096^3 +4.5 %, 6144^3 / 10240^3 +2 %),
+    # level with it on the large grids; the barrier inside the last k-step adds a little
+    form = 1.0
+    if getattr(cfg, "mfma", 32) == 16:
+        form = 1.02 + (0.004 if getattr(cfg, "early", 0) else 0.0)
+        # accumulators in accumulation registers: about 3 % over the builtin form (measured
+        # at 4096^3 and 8192^3)
+        if getattr(cfg, "agpr", False):
+            form += 0.03
+        # tile loads dealt over the MFMA groups: the more loads a wave issues per K-tile, the
+        # longer the queue at the load path that the burst form makes every wave stand in
+        # (measured with 8 loads per lane and K-tile: +2 % at 4096^3, +6 % at 8192^3, +7.5 %
+        # at 16384^3; with 4: +1 %)
+        if getattr(cfg, "spread", 0):
+            loads = (cfg.BM * cfg.BK + cfg.BK * cfg.BN) // 8 // cfg.threads
+            form += 0.005 * loads
+    return form
+
+
+def gemm_general_score(cfg, arch, M: int, N: int, K: int) -> float:
     """
-    Heuristic score of an FP16 MFMA GEMM config.
+    Heuristic score of an FP16 MFMA GEMM config, by its terms (`gemm_tc_score` puts measured
+    step times in their place where it has them).
 
     Per-CU time per FLOP of the main loop, as a roofline whose non-bottleneck
     terms only partially overlap:
@@ -232,10 +272,6 @@ def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
     """
     from deca_amd.kernels.gemm_hip import tile_grid
 
-    if getattr(cfg, "edge", False):
-        by_steps = gemm_edge_score(cfg, arch, M, N, K)
-        if by_steps is not None:
-            return by_steps
     wgs = gemm_tc_occupancy(cfg, arch)
     slots = arch.sm_nums * wgs
     rows, cols = tile_grid(cfg, M, N)
@@ -302,27 +338,46 @@ def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
     # MFMA issue stream (measured ~15% on MI355X)
     staged = 1.0 if cfg.direct else getattr(arch, "gemm_staged_fill_factor", 0.85)
 
-    # 16x16x32 tiles: measured ahead of the 32x32x16 twin where the grid is a single wave of
-    # workgroups or leaves a partial one (2048^3 +7 %, 4096^3 +4.5 %, 6144^3 / 10240^3 +2 %),
-    # level with it on the large grids; the barrier inside the last k-step adds a little
-    form = 1.0
-    if getattr(cfg, "mfma", 32) == 16:
-        form = 1.02 + (0.004 if getattr(cfg, "early", 0) else 0.0)
-        # accumulators in accumulation registers: about 3 % over the builtin form (measured
-        # at 4096^3 and 8192^3)
-        if getattr(cfg, "agpr", False):
-            form += 0.03
-        # tile loads dealt over the MFMA groups: the more loads a wave issues per K-tile, the
-        # longer the queue at the load path that the burst form makes every wave stand in
-        # (measured with 8 loads per lane and K-tile: +2 % at 4096^3, +6 % at 8192^3, +7.5 %
-        # at 16384^3; with 4: +1 %)
-        if getattr(cfg, "spread", 0):
-            loads = (cfg.BM * cfg.BK + cfg.BK * cfg.BN) // 8 // cfg.threads
-            form += 0.005 * loads
-
+    form = gemm_form_factor(cfg)
     # (tiles that reach over the edge of C compute more than the shape needs)
     useful = M * N / (grid * cfg.BM * cfg.BN)
     return useful * form * wave_eff * hiding * pipe * sync_eff * staged / ((t_flop + t_epi) / t_mma)
+
+
+def gemm_step_times_apply(arch, M: int, N: int) -> bool:
+    """Shapes whose tile bodies are ranked by `GEMM_STEP_TIMES`: no multiple of 256 both ways,
+    or fewer tiles of 256 x 256 than there are CUs."""
+    return bool(M % 256 or N % 256 or M * N < 256 * 256 * arch.sm_nums)
+
+
+def gemm_tc_score(cfg, arch, M: int, N: int, K: int) -> float:
+    """Score of an FP16 MFMA GEMM config, larger is faster.
+
+    Where the step times apply, a tile body that has them scores by them whether or not it is
+    an `edge` form (the two are the same code where the tile divides C).  Its forms that were
+    not measured over the range stand to the measured one as in `gemm_general_score`, another
+    ring depth at most level with it (128 x 128 x 64 on 14 shapes: 4 stages 0-8 % behind 3, 5
+    stages 0-10 %, where the general score has them up to 22 and 33 % ahead).  All other bodies
+    stay on the general score, which reads about a quarter lower: of 175 shapes on which one of
+    them came first by it, the measured bodies were level or ahead on 168."""
+    edge = getattr(cfg, "edge", False)
+    if not (edge or gemm_step_times_apply(arch, M, N)):
+        return gemm_general_score(cfg, arch, M, N, K)
+    by_steps = gemm_edge_score(cfg, arch, M, N, K) if edge else None
+    if by_steps is not None:
+        return by_steps
+    twin = gemm_measured_form(cfg)
+    if twin is None:
+        return gemm_general_score(cfg, arch, M, N, K)
+
+    def rest(c):
+        return gemm_general_score(c, arch, M, N, K) / gemm_form_factor(c)
+
+    whole = replace(cfg, tail=False)
+    ring = replace(whole, stages=twin.stages)
+    ratio = (gemm_form_factor(cfg) / gemm_form_factor(twin) * (rest(ring) / rest(twin))
+             * min(1.0, rest(whole) / rest(ring)) * (rest(cfg) / rest(whole)))
+    return gemm_edge_score(twin, arch, M, N, K) * ratio
 
 
 def rank_gemm_configs(configs, arch, M: int, N: int, K: int, top_n: int | None = None,
@@ -334,8 +389,6 @@ def rank_gemm_configs(configs, arch, M: int, N: int, K: int, top_n: int | None =
     be spent on the six orders of the one or two best tile sets."""
     ranked = sorted(configs, key=lambda c: gemm_tc_score(c, arch, M, N, K), reverse=True)
     if per_tile:
-        from dataclasses import replace
-
         seen, kept = {}, []
         for c in ranked:
             key = replace(c, raster=1, early=0, agpr=False, spread=0)

@@ -2,11 +2,14 @@
 configurations first.  Times are microseconds per launch on an MI355X, launches back to back
 over buffers larger than the caches, both configurations in turn in one process."""
 
+from dataclasses import replace
+
 import pytest
 
-from deca_amd import Solver
+from deca_amd import Solver, tuned
 from deca_amd.arch import MI355X
 from deca_amd.cost_model import CostModel as cm
+from deca_amd.kernels.gemm_hip import GemmConfig
 from kernel_cases import GEMM_EDGE_CASES
 
 ARCH = MI355X()
@@ -77,11 +80,30 @@ def test_every_valid_edge_form_can_be_ranked(M, N, K, cfg):
 
 
 def test_edge_score_counts_useful_work_only():
-    from dataclasses import replace
-
-    from deca_amd.kernels.gemm_hip import GemmConfig
-
     # a body without step times: half of the last row of tiles is outside of C
     cfg = GemmConfig(128, 128, 32, 64, 64, 3, 2, False, edge=True)
     full, cut = (cm.gemm_tc_score(cfg, ARCH, M, 2048, 512) for M in (2048, 1984))
     assert cut < full == cm.gemm_tc_score(replace(cfg, edge=False), ARCH, 2048, 2048, 512)
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 2048, 2048), (1024, 1024, 1024), (1536, 4096, 512), (5120, 576, 512)])
+def test_one_tile_has_one_score(M, N, K):
+    """With and without `edge`, where the tile divides C and the two are the same code, and the
+    solver has it once."""
+    configs = Solver.solve_gemm_tc(ARCH, M, N, K)
+    assert len({replace(c, edge=False) for c in configs}) == len(configs)
+    measured = [c for c in configs if not c.edge and cm.gemm_edge_score(c, ARCH, M, N, K) is not None
+                and cm.gemm_measured_form(c) == replace(c, edge=True)]
+    assert measured
+    for c in measured:
+        assert cm.gemm_tc_score(c, ARCH, M, N, K) == cm.gemm_tc_score(replace(c, edge=True), ARCH, M, N, K)
+
+
+@pytest.mark.parametrize("inputs", ["normal", "uniform"])
+def test_tuning_a_small_grid_measures_the_stored_winner(inputs):
+    """2048^3: 36 candidates at up to three tile orders per tile set, as its table entry was
+    tuned; the entry's four-stage ring is not among the edge forms."""
+    shape = (2048, 2048, 2048)
+    stored = tuned.lookup(tuned.make_key("GEMM", shape, inputs=inputs))
+    ranked = cm.rank_gemm_configs(Solver.solve_gemm_tc(ARCH, *shape), ARCH, *shape, top_n=36, per_tile=3)
+    assert stored in ranked
