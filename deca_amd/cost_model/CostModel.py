@@ -450,15 +450,19 @@ def fa_split_score(cfg, arch, shape, causal: bool = False) -> float:
         # (1.2: of 1.0 to 1.3 the factor that leaves the fewest slower choices over the shapes
         # below; at 1.0 there are two more)
         t = math.ceil(rounds) * longest * (1.2 if rounds > 1 else 1.0)
-    # From two rows of 32 queries per CU on the plain forms fill their SIMDs too, and the fewer
-    # keys, the more the meeting of the waves weighs.  Of 350 shapes (1 to 8 rows per CU, S_kv
-    # 256 ... 13504) 30 took up to 16 % longer than in the plain form without these two terms,
-    # most of them full ones with few keys and D 64 (B3 H16 S 384: 8.0 us instead of 7.1); with
-    # them 7, all but one by less than 9 %.
+    # From two rows of 32 queries per CU on the plain forms fill their SIMDs too: under the causal
+    # mask, whose rows differ in length, the more of them the better they do; without it the
+    # fewer keys there are, the more the meeting of the waves weighs.  Of 419 shapes (1 to 8 rows
+    # per CU, S_kv 256 ... 13504) 36 took up to 16 % longer than in the plain form without these
+    # two terms, most of them full ones with few keys and D 64 (B3 H16 S 384: 8.2 us instead of
+    # 7.1); with them 13, all but one by less than 10 %.  (The rows term on full shapes: 18 %
+    # lost on B1 H16 S_q 2624 S_kv 3776 D 64, nothing won.)
     rows = B * H * S_q / 32 / arch.sm_nums
-    gain = max(1.0, rows / 2) ** -0.15
-    if rows >= 2 and not causal:
-        gain *= min(1.0, S_kv * D / (1024 * 64)) ** 0.3
+    gain = 1.0
+    if causal:
+        gain = max(1.0, rows / 2) ** -0.15
+    elif rows >= 2:
+        gain = min(1.0, S_kv * D / (1024 * 64)) ** 0.3
     flops = 4.0 * B * H * S_q * S_kv * D * (0.5 if causal else 1.0)
     return gain * flops / (arch.peak_mma_sync_flops * 1e9) / ((t - launch) * (0.8 if causal else 0.95))
 

@@ -63,6 +63,7 @@ def test_attention_first_rank_is_not_the_slower_form(B, H, S_q, S_kv, D, causal,
 KEY_SPLIT = [
     (1, 16, 512, 512, 64, True), (1, 16, 512, 8192, 128, False), (4, 8, 320, 384, 64, False),
     (1, 8, 1216, 12096, 128, False), (2, 16, 768, 768, 64, True), (3, 16, 704, 704, 128, True),
+    (1, 16, 2624, 3776, 64, False),
 ]
 
 
