@@ -260,10 +260,15 @@ def solve_rowwise(
         # 16-byte accesses, with half a vector at the end.  From three vectors a lane: with two,
         # of which the second is part empty, 8-byte accesses are up to 18 % ahead (softmax bf16
         # 2713 x 4116 with 512 lanes: 10.4 and 11.7 us; RMSNorm bf16 20359 x 1044: 18.3 and 21.3).
+        # Two full to 0.9 are level or ahead from 96 KiB per CU on (RMSNorm bf16 17558 x 1988:
+        # 25.5 us, 26.7 with 8-byte accesses).
         longer = _rowwise_constraints(arch, op, M, N + 4, type_size, force_reg=True)
+        large = M * N * type_size >= 96 * 1024 * arch.sm_nums
         for tpr, rpb, vec, _, _, hint in _enumerate(ROWWISE_DOMAINS, longer, count, backend):
+            two = 2 * tpr * vec
             # (several rows a workgroup: from two workgroups per CU; 512 x 50004 loses 12 %)
-            if vec == 8 and 2 * tpr * vec < N and (rpb == 1 or M // rpb >= 2 * arch.sm_nums):
+            if (vec == 8 and (N > two or (large and N >= 0.9 * two))
+                    and (rpb == 1 or M // rpb >= 2 * arch.sm_nums)):
                 configs.append(RowConfig(threads_per_row=tpr, rows_per_block=rpb, vec=8,
                                          hint=bool(hint), half=True))
     return configs[:count]

@@ -22,6 +22,8 @@ ROWWISE = [
     ("softmax", 6309, 564, "tpr=64,rpb=1,vec=8,mode=reg,hint=1,half=1", 5.4, 4.9),
     ("rmsnorm", 20359, 1044, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 21.3, 18.3),
     ("rmsnorm", 611, 4820, "tpr=512,rpb=1,vec=8,mode=reg,hint=1,half=1", 4.5, 4.2),
+    # ... which is nearly full here
+    ("rmsnorm", 17558, 1988, "tpr=128,rpb=2,vec=4,mode=reg,hint=1", 26.7, 25.5),
     # rows all resident at once: several rows a workgroup, fewer lanes than a wave or 8-byte
     # accesses have nothing of what one wave a row gains there, nor has it with long softmax rows
     ("softmax", 7338, 3000, "tpr=32,rpb=2,vec=8,mode=reg,hint=1", 18.2, 17.0),
