@@ -189,10 +189,20 @@ GEMM_EDGE_CASES = [
     (128, 128, 256, GemmConfig(64, 64, 64, 32, 32, 3, 1, True, mfma=16, kgroups=2, xcd=False)),
 ]
 
+# the same in bf16, as the solver chooses them: wave groups with and without an edge, the 128 x
+# 128 body, and the direct-store epilogue
+GEMM_EDGE_BF16_CASES = [
+    (256, 256, 1152, GemmConfig(64, 64, 128, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
+    (100, 136, 512, GemmConfig(64, 64, 128, 64, 32, 3, 1, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
+    (255, 504, 192, GemmConfig(128, 128, 64, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, edge=True)),
+    (257, 264, 128, GemmConfig(256, 256, 64, 128, 64, 2, 2, True, mfma=16, early=4, agpr=True, spread=6, edge=True)),
+    (512, 712, 256, GemmConfig(128, 64, 64, 64, 32, 3, 1, False, mfma=16, early=2, agpr=True, edge=True)),
+]
+
 
 def gemm_specs():
     return ([make_gemm_tc(M, N, K, cfg) for M, N, K, cfg in GEMM_CASES + GEMM_EDGE_CASES + GEMM_FULL] +
-            [make_gemm_tc(M, N, K, cfg, "bfloat16") for M, N, K, cfg in GEMM_BF16_CASES])
+            [make_gemm_tc(M, N, K, cfg, "bfloat16") for M, N, K, cfg in GEMM_BF16_CASES + GEMM_EDGE_BF16_CASES])
 
 
 # (B, H, S_q, S_kv, D, causal, cfg): sizes the CPU checker finishes in seconds
