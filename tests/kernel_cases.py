@@ -393,7 +393,8 @@ SOLVER_FA_SHAPES = [(2, 16, 1024, 64, False), (2, 16, 1024, 64, True), (2, 16, 1
                     (2, 16, 1024, 192, True)]
 SOLVER_GEMM_SHAPES = [(2048, 2048, 2048), (3072, 3072, 512)]  # the second leaves partial waves (tail)
 SOLVER_ROW_SHAPES = [("softmax", 2048, 4096, "float16"), ("rmsnorm", 2048, 8192, "bfloat16"),
-                     ("softmax", 512, 32000, "float16"), ("rmsnorm", 512, 128256, "float16")]
+                     ("softmax", 512, 32000, "float16"), ("rmsnorm", 512, 128256, "float16"),
+                     ("softmax", 777, 6020, "bfloat16")]  # the last: half-vector forms among them
 SAMPLE = 24
 
 

@@ -175,3 +175,24 @@ def test_launch_rejects_wrong_arguments():
         kern(x)  # missing output
     with pytest.raises(ValueError):
         kern(x.cpu(), x)  # host tensor
+
+
+@pytest.mark.parametrize("op,M,N,dtype,cfg", [c for c in ROWWISE_CASES if c[-1].half], ids=lambda v: str(v))
+def test_half_vector_rows_end_where_they_end(op, M, N, dtype, cfg):
+    """Elements behind the last row stay as they are (a whole vector stored at its end would
+    reach them), and NaN there does not come into the row."""
+    from deca_amd.kernels.rowwise_hip import build_rowwise, make_rowwise
+
+    print(f"case {op} {M}x{N} {dtype} {cfg} with a guard", flush=True)
+    inputs = _inputs(op, M, N, dtype, seed=M + N)
+    dev = []
+    for t in inputs:
+        padded = torch.full((t.numel() + 64,), float("nan"), dtype=t.dtype, device="cuda")
+        padded[:t.numel()] = t.cuda().flatten()
+        dev.append(padded[:t.numel()].view(t.shape))
+    out = torch.full((M * N + 64,), 7.0, dtype=inputs[0].dtype, device="cuda")
+    kern = build_rowwise(make_rowwise(op, M, N, dtype, cfg, EPS))
+    kern(*dev, out[:M * N].view(M, N))
+    torch.cuda.synchronize()
+    assert bool((out[M * N:] == 7.0).all())
+    _check(op, dtype, out[:M * N].view(M, N).cpu(), inputs)
