@@ -161,3 +161,74 @@ def test_tuner_end_to_end(arch, operator, shape, kw):
     unit = "GB/s" if operator == "softmax" else "TFLOPS"
     assert re.search(rf"throughput: \d+\.\d {unit} \(\d+% of ", text)
     assert os.environ.get("HIP_VISIBLE_DEVICES", "0") is not None
+
+
+def test_launches_follow_the_callers_stream_and_thread():
+    """A call launches on the stream that is current in the calling thread: behind work queued
+    there (on another stream it would read the input before that work has written it), and two
+    threads with a stream each do not mix."""
+    import threading
+
+    from deca_amd.kernels.rowwise_hip import RowConfig, build_rowwise, make_rowwise
+
+    M, N = 2048, 4096
+    kern = build_rowwise(make_rowwise("softmax", M, N, "float16", RowConfig(128, 1, 8)))
+    big = torch.randn(4096, 4096, device="cuda")
+    source = [torch.randn(M, N, device="cuda").half() for _ in range(2)]
+    want = [torch.softmax(x.float(), -1) for x in source]
+    stale = torch.zeros(M, N, dtype=torch.float16, device="cuda")
+    results, errors = {}, []
+    torch.cuda.synchronize()
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                assert kern._stream() == stream.cuda_stream
+                x, y = stale.clone(), torch.empty_like(stale)
+                for r in range(8):
+                    x.zero_()
+                    for _ in range(4):
+                        torch.mm(big, big)  # keeps this stream busy while the next calls are queued
+                    x.copy_(source[i])
+                    kern(x, y)
+                    results[i, r] = y.clone()
+                stream.synchronize()
+        except Exception as err:  # noqa: BLE001
+            errors.append(err)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not errors and len(results) == 16
+    torch.cuda.synchronize()
+    assert kern._stream() == torch.cuda.current_stream().cuda_stream
+    for (i, _), y in results.items():
+        assert (y.float() - want[i]).abs().max().item() <= 2e-3
+
+
+def test_prepared_launch_in_a_graph():
+    """The launch path of a call can be captured, and replays read the buffers' new contents."""
+    from deca_amd.kernels.rowwise_hip import RowConfig, build_rowwise, make_rowwise
+
+    M, N = 512, 4096
+    kern = build_rowwise(make_rowwise("softmax", M, N, "float16", RowConfig(128, 1, 8)))
+    x = torch.randn(M, N, device="cuda").half()
+    y = torch.empty_like(x)
+    kern(x, y)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kern(x, y)
+    for seed in range(3):
+        torch.manual_seed(seed)
+        x.copy_(torch.randn(M, N, device="cuda").half())
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = y.clone()
+        kern(x, y)
+        torch.cuda.synchronize()
+        assert torch.equal(got, y)
