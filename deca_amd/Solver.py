@@ -437,8 +437,10 @@ def _edge_forms(arch, M: int, N: int, K: int):
         rows, cols = tile_grid(cfg, M, N)
         # A single round that leaves CUs idle: where smaller tiles come out even (multiples of
         # 256) it loses from 30 % on, elsewhere it may still win at half (1664 x 640: 130 tiles
-        # of 64 x 128 against 260 of 64 x 64).  Wave groups pay while they are a CU's only
-        # waves (512 x 4096, two tiles per CU: the plain 64 x 128 tile is 10-20 % ahead).
+        # of 64 x 128 against 260 of 64 x 64).  Wave groups pay in a single round, with rings that
+        # leave a CU room for one tile: 64 x 64 tiles at exactly one per CU, which is the smallest
+        # M * N that has a config, the 64 x 128 and 128 x 64 ones up to twice that (2 ... 11 % over
+        # the plain tiles on 15 of 15 shapes with K from 1280; beyond one round 15 ... 40 % behind).
         if rows * cols < (0.7 if even else 0.5) * arch.sm_nums or (kg > 1 and rows * cols > arch.sm_nums):
             continue
         for ras in GEMM_RASTERS:

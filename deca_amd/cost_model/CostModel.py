@@ -161,22 +161,27 @@ def gemm_mma_peak(cfg, arch) -> float:
     return arch.peak_mma_sync_flops
 
 
-# Measured times of the eight-wave tile bodies (16x16x32 tiles, accumulators in AGPRs where
-# they fit, load window): (BM, BN, BK, warp_m, warp_n, stages, kgroups) -> microseconds of
-# (a workgroup's prologue and epilogue, one K-tile of a workgroup alone on its CU, one K-tile
-# of each of two on a CU).  Fitted to seven shapes that are multiples of 64 and of little else
-# (M 704 ... 4800, N 640 ... 7360, K 512 ... 5440); the times these give are within 10 % there.
+# Step times of the tile bodies (16x16x32 tiles, accumulators in AGPRs where they fit, load
+# window): (BM, BN, BK, warp_m, warp_n, stages, kgroups) -> microseconds of (a workgroup's
+# prologue and epilogue, one K-tile of a workgroup alone on its CU, one K-tile of each of two on
+# a CU; None where the LDS ring leaves room for one only).  Fitted to the times of seven shapes
+# that are multiples of 64 and of little else (M 704 ... 4800, N 640 ... 7360, K 512 ... 5440),
+# within 10 % there; those of the wave groups (kgroups = 2) to 1024^3 and 256 x 4096 x 4096 (the
+# 64 x 64 tile) and to what the other two gain over the plain tile of their size on 22 shapes of
+# up to one tile per CU (K 512 ... 1024: -3 ... +5 %, 1280 ... 7936: 2-11 %).
 # What they show is the CU's load path and the fabric behind its L2 rather than the matrix pipe:
 # 32 KiB per 128 x 128 K-tile at 70 KB/us and CU.
 GEMM_STEP_TIMES = {
-    (256, 256, 64, 128, 64, 2, 1): (6.0, 1.154, 2.308),
-    (256, 128, 64, 64, 64, 3, 1): (2.6, 0.776, 1.552),
-    (128, 256, 64, 64, 64, 3, 1): (2.7, 0.757, 1.514),
-    (128, 128, 64, 64, 32, 3, 1): (1.3, 0.476, 0.952),
+    (256, 256, 64, 128, 64, 2, 1): (6.0, 1.154, None),
+    (256, 128, 64, 64, 64, 3, 1): (2.6, 0.776, None),
+    (128, 256, 64, 64, 64, 3, 1): (2.7, 0.757, None),
+    (128, 128, 64, 64, 32, 3, 1): (1.3, 0.476, None),
     (128, 64, 64, 64, 32, 3, 1): (1.0, 0.304, 0.594),
     (64, 128, 64, 64, 32, 3, 1): (1.0, 0.301, 0.597),
     (64, 64, 64, 32, 32, 5, 1): (1.0, 0.225, 0.390),
-    (64, 64, 128, 64, 32, 3, 2): (1.0, 0.410, 0.820),
+    (128, 64, 128, 64, 32, 3, 2): (1.4, 0.558, None),
+    (64, 128, 128, 64, 32, 3, 2): (1.4, 0.556, None),
+    (64, 64, 128, 64, 32, 3, 2): (1.0, 0.410, None),
 }
 
 

@@ -23,13 +23,15 @@
 //                 per K-tile at 70 KB/us and CU (L2 hits and the fabric behind the L2)
 //   DECA_KGROUPS  n > 1 (16x16x32 body): n groups of waves each hold all of the tile's
 //                 accumulators and take 1 / n of the k-steps of every K-tile; their sums
-//                 meet in LDS at the end (fp32).  For 64 x 64 tiles, of which a CU of a
-//                 256-workgroup grid has one: with K-tiles of 128 and two groups of 64 x 32
-//                 wave tiles there are half as many barriers and three quarters of the LDS
-//                 reads (compute side alone, four waves of 32 x 32 and K-tiles of 64: 547
-//                 clocks per K-tile for 128 of matrix work).  1024^3 fp16: 6.0 -> 4.8 us,
-//                 256 x 4096 x 4096 bf16: 16.9 -> 15.2 us; the loads alone (128 KiB in
-//                 flight, 1 MiB per CU from L2) take 15.5 us of the latter
+//                 meet in LDS at the end (fp32).  For tiles of which a CU has one: with
+//                 K-tiles of 128 and two groups of 64 x 32 wave tiles there are half as many
+//                 barriers, and for 64 x 64 tiles three quarters of the LDS reads of four
+//                 waves of 32 x 32 (compute side of those alone: 547 clocks per 64-deep
+//                 K-tile for 128 of matrix work).  64 x 64 tiles: 1024^3 fp16 6.0 -> 4.8 us,
+//                 256 x 4096 x 4096 bf16 16.9 -> 15.2 us, of which the operands alone, 1 MiB
+//                 per CU, take about all (15.5 us through the 64-deep ring of that size).
+//                 128 x 64 and 64 x 128 tiles, twice the waves: 1344 x 1088 x 2944 fp16
+//                 15.8 -> 14.5 us, 512 x 2880 x 7936 bf16 37.8 -> 34.2 us
 //   DECA_DIRECT   1: global -> LDS loads that bypass the VGPRs, ring of
 //                 DECA_STAGES (2..5) tiles; 0: loads staged through VGPRs one
 //                 tile ahead, ring of 1 or 2 tiles

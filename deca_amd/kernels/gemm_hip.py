@@ -79,8 +79,8 @@ class GemmConfig:
     # last row and column of tiles reach over the edge of C
     edge: bool = False
     # 16x16x32 body: groups of waves that share the k-steps of a K-tile, each with all of the
-    # tile's accumulators; the sums meet in LDS (fp32).  More waves per SIMD and fewer barriers
-    # (K-tiles of 128) for tiles too small to fill a CU's SIMDs
+    # tile's accumulators; the sums meet in LDS (fp32).  With K-tiles of 128 half the barriers
+    # per k, for tiles that a CU has only one of
     kgroups: int = 1
 
     @property

@@ -187,6 +187,8 @@ GEMM_EDGE_CASES = [
     (256, 264, 256, GemmConfig(128, 128, 64, 64, 64, 3, 1, True, mfma=16, early=2, agpr=True, kgroups=2, edge=True)),
     (192, 128, 512, GemmConfig(64, 64, 128, 32, 32, 4, 3, True, mfma=16, agpr=True, xcd=False)),
     (128, 128, 256, GemmConfig(64, 64, 64, 32, 32, 3, 1, True, mfma=16, kgroups=2, xcd=False)),
+    (129, 72, 384, GemmConfig(128, 64, 128, 64, 32, 3, 2, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
+    (320, 1088, 640, GemmConfig(64, 128, 128, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
 ]
 
 # the same in bf16, as the solver chooses them: wave groups with and without an edge, the 128 x
@@ -194,6 +196,8 @@ GEMM_EDGE_CASES = [
 GEMM_EDGE_BF16_CASES = [
     (256, 256, 1152, GemmConfig(64, 64, 128, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
     (100, 136, 512, GemmConfig(64, 64, 128, 64, 32, 3, 1, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
+    (320, 1088, 640, GemmConfig(128, 64, 128, 64, 32, 3, 2, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
+    (193, 328, 384, GemmConfig(64, 128, 128, 64, 32, 3, 2, True, mfma=16, early=2, agpr=True, spread=3, kgroups=2, edge=True)),
     (255, 504, 192, GemmConfig(128, 128, 64, 64, 32, 3, 4, True, mfma=16, early=2, agpr=True, spread=3, edge=True)),
     (257, 264, 128, GemmConfig(256, 256, 64, 128, 64, 2, 2, True, mfma=16, early=4, agpr=True, spread=6, edge=True)),
     (512, 712, 256, GemmConfig(128, 64, 64, 64, 32, 3, 1, False, mfma=16, early=2, agpr=True, edge=True)),

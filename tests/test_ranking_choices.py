@@ -110,3 +110,14 @@ def test_tuning_a_small_grid_measures_the_stored_winner(inputs):
     stored = tuned.lookup(tuned.make_key("GEMM", shape, inputs=inputs))
     ranked = cm.rank_gemm_configs(Solver.solve_gemm_tc(ARCH, *shape), ARCH, *shape, top_n=36, per_tile=3)
     assert stored in ranked
+
+
+# a single round of 128 x 64 or 64 x 128 tiles: wave groups were measured 4 ... 11 % ahead
+KGROUPS = [(640, 1792, 2048), (1344, 1088, 2944), (2304, 704, 3072), (896, 1792, 5760),
+           (1664, 1024, 7168), (512, 2880, 7936), (320, 3392, 1280)]
+
+
+@pytest.mark.parametrize("M,N,K", KGROUPS)
+def test_gemm_wave_groups_serve_the_grids_of_one_round(M, N, K):
+    first = cm.rank_gemm_configs(Solver.solve_gemm_tc(ARCH, M, N, K), ARCH, M, N, K)[0]
+    assert first.kgroups == 2 and -(-M // first.BM) * -(-N // first.BN) <= ARCH.sm_nums
