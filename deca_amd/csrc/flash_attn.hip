@@ -551,9 +551,9 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   // first key of this wave's tile j
   auto key0 = [&](int j) __attribute__((always_inline)) { return (j * KVG + kvg) * BC; };
   auto nothing = [](int) __attribute__((always_inline)) {};
-  // Causal mask of tile j.  Only tiles crossing the diagonal need it; every
-  // query sees key 0 in tile 0, so its running max is finite before a fully
-  // masked block shows up.
+  // Causal mask of tile j.  Only tiles crossing the diagonal need it.  A wave that takes every
+  // tile has seen key 0 in tile 0, so that its running max is a score before a fully masked
+  // block shows up; one with a share of the keys may not have (see M_START).
   auto mask_s = [&](acc_t (&s_acc)[KT][MQ], int j) __attribute__((always_inline)) {
 #if DECA_CAUSAL
     if (key0(j) + BC - 1 > qt * BR + qw * WQ) {
