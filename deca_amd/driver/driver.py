@@ -14,7 +14,7 @@ import ctypes
 import os
 from ctypes import POINTER, byref, c_char, c_char_p, c_float, c_int, c_size_t, c_uint, c_void_p
 
-from deca_amd.driver.build_lib import LIB_PATH
+from deca_amd.driver.build_lib import EXT_PATH, LIB_PATH
 
 
 class DevInfo(ctypes.Structure):
@@ -230,17 +230,22 @@ def get_driver() -> HipDriver:
     return _driver
 
 
-def _raw_stream_query():
-    """torch's query of the current stream's handle without a Stream object around it, where
-    this torch has it (`torch.cuda.current_stream()` costs 2.9 us a call, this 0.2)."""
+def _load_launch():
+    """`_launch.launch` of the extension module, None where there is no torch (whose tensors it
+    takes): then only the pointer interface of this file works."""
     try:
-        from torch._C import _cuda_getCurrentRawStream as stream_of, _cuda_getDevice as device
+        import torch  # noqa: F401
     except ImportError:
         return None
-    return lambda: stream_of(device())
+    if not os.path.exists(EXT_PATH):
+        raise RuntimeError(
+            f"{EXT_PATH} is missing: build it with `python -m deca_amd.driver.build_lib`")
+    from deca_amd._launch import launch
+
+    return launch
 
 
-_raw_stream = None  # set with the first kernel that is loaded (torch is not imported before)
+_launch = None  # set with the first kernel that is loaded (torch is not imported before)
 
 
 class KernelRejected(RuntimeError):
@@ -261,17 +266,16 @@ class LoadedKernel:
         self.launches = 0  # launches issued through this object so far
         self.drv = get_driver()
         self.drv.init(device)
-        global _raw_stream
-        if _raw_stream is None:
-            _raw_stream = _raw_stream_query()
+        global _launch
+        if _launch is None:
+            _launch = _load_launch()
         self.mod = self.drv.module_load(path)
         self.fn = self.drv.get_function(self.mod, spec.symbol)
         # every kernel of this package takes at most four pointers (`launch` takes any)
-        self._plan = self._call_plan = None
-        if 1 <= spec.nargs <= LaunchPlan.MAX_ARGS:
+        self._plan, self._plan_address = None, 0
+        if _launch is not None and 1 <= spec.nargs <= LaunchPlan.MAX_ARGS:
             self._plan = LaunchPlan(self.fn, spec.grid, spec.block, spec.lds_bytes, spec.nargs)
-            self._call_plan = (self.drv.lib.deca_launch_plan, byref(self._plan),
-                               (None,) * (LaunchPlan.MAX_ARGS - spec.nargs))
+            self._plan_address = ctypes.addressof(self._plan)
         if spec.lds_bytes > 64 * 1024:
             self.drv.set_max_dynamic_lds(self.fn, spec.lds_bytes)
         # A kernel whose loop waits for "all but the newest n" of its global->LDS loads
@@ -294,8 +298,6 @@ class LoadedKernel:
     @staticmethod
     def _stream() -> int:
         """Handle of torch's current stream of the current device."""
-        if _raw_stream is not None:
-            return _raw_stream()
         import torch
 
         return int(torch.cuda.current_stream().cuda_stream)
@@ -309,16 +311,18 @@ class LoadedKernel:
         return [t.data_ptr() for t in tensors]
 
     def __call__(self, *tensors):
-        # The host's share of a launch: of 7.8 us (2.9 for a torch Stream object, the rest
-        # mostly argument conversion) 3.9 remain; the smallest kernels take 2.6.
+        # The host's share of a launch: 3.9 us with the checks in Python and a foreign-function
+        # call, 3.2 with both in one C function, of which the runtime's own launch takes 2.7
+        # (softmax 256 x 1024, whose kernel takes 2.1: 4.3 -> 3.1 us a call; GEMM 1024^3
+        # 5.5 -> 4.4, bound by its kernel).
         self.launches += 1
-        if self._call_plan is not None:
-            entry, plan, unused = self._call_plan
-            ptrs = self._ptrs(tensors)  # (checks them: device tensors, so that torch's runtime is up)
-            code = entry(plan, self._stream(), *ptrs, *unused)
-            if code:
+        if self._plan_address:
+            code = _launch(self._plan_address, *tensors)
+            if code == 0:
+                return
+            if code > 0:
                 self.drv.check(code, "deca_launch_plan")
-            return
+            # (an argument it cannot take: named by the checks below)
         self.drv.launch(
             self.fn, self.spec.grid, self.spec.block, self.spec.lds_bytes, self._stream(),
             self._ptrs(tensors),
