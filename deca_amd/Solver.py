@@ -463,6 +463,15 @@ FA_DOMAINS = {
     "mfma": (32, 16),  # 16: v_mfma_f32_16x16x32 tiles (plain and slot loop)
     "qs": (0, 1),  # Q tile staged in LDS and re-read every KV step (Solver.py:335)
 }
+# Query tiles that need not divide S_q (`FAConfig.edge`): a sequence that is an odd multiple of 64
+# otherwise only has tiles of 64 rows, whose two waves each bring in all of K and V.  On 25 of 26
+# such shapes the best of them was 5 ... 51 % ahead (B4 H8 S 3392 D 64: 135 -> 106 us; B9 H16 S 576
+# D 128 causal: 1.4x).  Not for multiples of 128 (tiles of 256: 4 ... 24 % behind on 6 of 8), nor below
+# the stated rows of 32 queries per CU, where the tiles are too few (0.8 ... 1.2x on six shapes), nor
+# with less than the stated share of the rows in the sequence.
+FA_EDGE_BR = (128, 256)
+FA_EDGE_MIN_FILL = 0.6
+FA_EDGE_MIN_ROWS_PER_CU = 5.25
 # `swizzle` stays out of the search (the reference enumerates it, Solver.py:336): linear LDS
 # rows are never faster here, `FAConfig(swizzle=False)` exists for the comparison only.
 
@@ -551,10 +560,18 @@ def solve_flash_attn(arch, B: int, H: int, S_q: int, S_kv: int, D: int, type_siz
     from deca_amd.kernels.flash_attn_hip import default_spread, register_fill
 
     cons = _fa_constraints(arch, B, H, S_q, S_kv, D, type_size, max_est_regs)
+    tiles = [(t, False) for t in _enumerate(FA_DOMAINS, cons, count, backend)]
+    odd = S_q % 128 and S_q % 32 == 0 and B * H * S_q // 32 >= FA_EDGE_MIN_ROWS_PER_CU * arch.sm_nums
+    for br in FA_EDGE_BR if odd else ():
+        # tiles that reach over the end of the query sequence: those of the next longer one
+        if S_q >= FA_EDGE_MIN_FILL * (longer := -(-S_q // br) * br):
+            cons = _fa_constraints(arch, B, H, longer, S_kv, D, type_size, max_est_regs)
+            tiles += [(t, True) for t in _enumerate({**FA_DOMAINS, "br": (br,), "pipe": (0, 2)}, cons,
+                                                    count, backend)]
     results = []
-    for br, bc, nw, st, pipe, mfma, qs in _enumerate(FA_DOMAINS, cons, count, backend):
+    for (br, bc, nw, st, pipe, mfma, qs), edge in tiles:
         cfg = FAConfig(Br=br, Bc=bc, num_warps=nw, stages=st, pipe=int(pipe), mfma=mfma,
-                       q_in_smem=bool(qs))
+                       q_in_smem=bool(qs), edge=edge)
         forms = [cfg]
         # the plain ring loop in its one-copy form, where the unrolled one is expected to
         # run out of registers (it interacts with no other constraint: expanded here)

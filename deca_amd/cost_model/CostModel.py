@@ -493,7 +493,10 @@ def fa_score(cfg, arch, shape, causal: bool = False) -> float:
     if getattr(cfg, "kv_split", False):
         return fa_split_score(cfg, arch, shape, causal)
     B, H, S_q, S_kv, D = shape
-    grid = (S_q // cfg.Br) * B * H
+    from deca_amd.kernels.flash_attn_hip import query_tiles
+
+    nq = query_tiles(cfg, S_q)
+    grid = nq * B * H
     wgs, _ = fa_occupancy(cfg, arch, D, grid)
     slots = arch.sm_nums * wgs
     wave_eff = _wave_efficiency(grid, slots)
@@ -574,13 +577,12 @@ def fa_score(cfg, arch, shape, causal: bool = False) -> float:
     # statistics inside the matrix work and pays a little less of it
     step = 1.0 / (1.0 + (0.06 if int(cfg.pipe) == 2 else 0.08) * 64 / cfg.Bc)
 
-    useful = 1.0
+    useful = S_q / (nq * cfg.Br)  # (`edge`: rows beyond the sequence are computed for nothing)
     if causal:
         # a wave computes every tile that reaches one of its rows in full and skips the
         # tiles beyond its last row
-        nq = S_q // cfg.Br
-        computed = sum(-(-(i * cfg.Br + (w + 1) * wq) // cfg.Bc) * cfg.Bc * wq
-                       for i in range(nq) for w in range(cfg.num_warps))
+        # (`edge`: a wave whose rows all lie beyond the sequence computes nothing)
+        computed = sum(-(-min(r + wq, S_kv) // cfg.Bc) * cfg.Bc * wq for r in range(0, S_q, wq))
         useful = S_q * (S_q + 1) / 2 / computed
         # The workgroups of a causal launch differ in length, and towards the end many CUs
         # hold a single one.  A workgroup that fills its SIMDs with two waves by itself keeps
@@ -610,7 +612,146 @@ def fa_score(cfg, arch, shape, causal: bool = False) -> float:
     return wave_eff * pipe * sync * step * useful * chain * ramp / (t_flop / t_mma)
 
 
+# Coefficients of `fa_time`, in microseconds where they are times, for head dim 128 where they are
+# multiplied by D / 128.  Least squares on the logarithm of 4834 measured times (launches back to
+# back over buffers larger than the caches) of 357 shapes: 0.5 to 120 rows of 32 queries per CU,
+# S_q 128 ... 8192, S_kv 256 ... 15104, D 64 and 128, full and causal, nearly all drawn at random;
+# the configurations near a shape's best count most.
+FA_TIME = {
+    # one 32 x 32 block of scores in a wave's own chain of instructions (matrix and vector part),
+    # and its share of a SIMD that has other waves to fill the gaps
+    "chain_mfma": 0.36, "chain_valu": 0.0417, "busy_mfma": 0.185, "busy_valu": 0.123,
+    # of one key step: barrier and first fragments (workgroups of eight waves need a tenth of
+    # it), the wait for a tile in a one-slot ring, and of that where waves split the keys
+    "step": 0.145, "step_8_waves": 0.2, "one_slot": 0.381, "one_slot_split": 0.0664,
+    # a 32-key tile on the CU's load path; per wave where waves split the keys
+    "load": 0.109, "load_split": 0.15,
+    "overlap": 2.2,  # exponent that joins chain, busy pipes and load path into a step's time
+    # per workgroup: fixed, per 32 query rows of a wave, per 32 keys of a tile (the first one is
+    # waited for), without a second workgroup beside it (per wave), and the meeting of the waves
+    # that split keys (per wave; less under the mask); more where more workgroups share the CU
+    "wg": 0.379, "wg_rows": 2.22, "wg_tile": 0.2, "wg_alone": 0.362,
+    "meet": 0.25, "meet_causal": -0.305, "wg_shared": 0.254, "meet_shared": 0.208,
+    # a part-filled last round counts for this share of a round (a little less where several
+    # workgroups share a CU); under the mask, exponent that joins the sum of the work and the
+    # longest row of it
+    "round": 0.636, "round_shared": -0.076, "causal": 2.73,
+    # memory: bytes at 6.4 TB/s times this, joined by this exponent; the launch
+    "memory": 1.19, "memory_join": 1.5, "launch": 0.732,
+}
+# Logarithms of what the form of a key step does to its time; held near the medians over pairs of
+# configurations that differ in nothing else.
+FA_FORM = {
+    "mfma16_64": 0.0463, "mfma16_128": 0.0931, "mfma16_slots": 0.0946, "mfma16_causal": -0.054,
+    "mfma16_roll": -0.0271, "slots_causal": -0.0577, "trust_causal": 0.0693, "trust_mfma16_64": -0.0515,
+    "three_slots": 0.135, "three_slots_64": -0.046, "three_slots_large": 0.03,
+    "q_lds": 0.0982, "q_lds_64": -0.0584, "spread": 0.0146, "spread_slots": -0.116,
+    "spread_slots_64": 0.0794, "edge": -0.0406, "two_waves": 0.0582, "split_8": 0.0679,
+    "split_8_causal": 0.059,
+}
+
+
+def fa_form_factor(cfg, D: int, causal: bool) -> float:
+    """What the form of a key step (`FA_FORM`) does to its time."""
+    f, small, full = FA_FORM, D < 128, not causal
+    mfma16, slots = cfg.mfma == 16, int(cfg.pipe) == 2
+    log = 0.0
+    if mfma16:
+        log += f["mfma16_64"] if small else f["mfma16_128"]
+        log += f["mfma16_slots"] * slots + f["mfma16_causal"] * causal + f["mfma16_roll"] * cfg.roll
+    log += f["slots_causal"] * (slots and causal)
+    if cfg.trust:
+        log += f["trust_causal"] * causal + f["trust_mfma16_64"] * (full and mfma16 and small)
+    if cfg.stages == 3:
+        log += (f["three_slots"] + f["three_slots_64"] * small
+                + f["three_slots_large"] * (cfg.Bc * D > 32 * 128))
+    if cfg.q_in_smem:
+        log += f["q_lds"] + f["q_lds_64"] * small
+    if cfg.spread:
+        log += f["spread"] + (f["spread_slots"] + f["spread_slots_64"] * small) * slots
+    log += f["edge"] * cfg.edge
+    if cfg.kv_split:
+        log += (f["split_8"] + f["split_8_causal"] * causal) * (cfg.num_warps > 4)
+    else:
+        log += f["two_waves"] * (cfg.num_warps == 2)
+    return math.exp(log)
+
+
+def fa_time(cfg, arch, shape, causal: bool = False) -> float:
+    """Expected microseconds of a launch, head dims 64 and 128.
+
+    A workgroup is a number of key steps and a fixed part.  A step takes as long as its wave's own
+    chain of instructions, or as the busy pipes of a SIMD that its waves share, or as the CU's load
+    path, and somewhat longer where two of them are close.  All workgroups at once if they fit the
+    CUs; else rounds of those that do, of which a part-filled last one costs more than its share;
+    under the causal mask the sum of the work or the longest row, which starts first.
+    Of the 357 shapes the first choice by it is 3.0 % behind the best measured one on the average,
+    12 of them more than 16 % (39 % at most); with three quarters of the shapes in the fit 2.8 %
+    there and 3.5 % on the others.  By `fa_score`, which prices rounds of workgroups as if they kept
+    in step and knows no query edge, it is 7.4 % (80 % at most; 15 % from 8 rows of 32 queries per
+    CU on)."""
+    from deca_amd.kernels.flash_attn_hip import query_tiles
+
+    c = FA_TIME
+    B, H, S_q, S_kv, D = shape
+    d, split = D / 128, cfg.kv_split
+    grid = query_tiles(cfg, S_q) * B * H
+    fit, _ = fa_occupancy(cfg, arch, D, grid)
+    per_cu = grid / arch.sm_nums
+    most = math.ceil(per_cu)
+    together = min(most, fit)
+    mq, bc = cfg.wave_rows / 32, cfg.Bc / 32
+    steps = math.ceil(S_kv / (cfg.Bc * cfg.num_warps)) if split else S_kv / cfg.Bc
+    form = fa_form_factor(cfg, D, causal)
+    one_slot = c["one_slot_split" if split else "one_slot"] * (cfg.stages == 1)
+
+    def step(workgroups):
+        waves = workgroups * cfg.num_warps / arch.simds_per_cu
+        # (a single round is as long as its fullest SIMD)
+        waves = max(1.0, math.ceil(waves) if per_cu <= fit and workgroups > 1 else waves)
+        chain = (mq * bc * (c["chain_mfma"] * d + c["chain_valu"])
+                 + c["step"] * (c["step_8_waves"] if cfg.num_warps > 4 else 1.0) + one_slot)
+        busy = waves * mq * bc * (c["busy_mfma"] * d + c["busy_valu"])
+        load = (c["load_split"] * cfg.num_warps if split else c["load"]) * workgroups * bc * d
+        p = c["overlap"]
+        return (chain**p + busy**p + load**p) ** (1 / p) * form
+
+    fixed = c["wg"] + c["wg_rows"] * mq * d
+    fixed += c["meet"] * cfg.num_warps * d * mq if split else c["wg_tile"] * bc * d
+    fixed *= 1.0 + c["meet_shared" if split else "wg_shared"] * (together - 1)
+    if fit == 1 and most > 1 and not split:
+        fixed += c["wg_alone"] * cfg.num_warps * d
+    if split and causal:
+        fixed += c["meet_causal"]
+    rounds = per_cu / together
+    if causal:
+        mean = steps * 0.5 * (1.0 + cfg.Br / S_q) * step(together) + fixed
+        longest = steps * 0.5 * (step(1) + step(together)) + fixed
+        q = c["causal"]
+        t = ((rounds * mean) ** q + longest**q) ** (1 / q)
+    else:
+        t = steps * step(together) + fixed
+        if most > fit:
+            t *= ((1.0 - c["round"]) * rounds + c["round"] * math.ceil(rounds)
+                  + c["round_shared"] * (fit > 1))
+    memory = c["memory"] * 2 * B * H * D * 2 * (S_q + S_kv) / 6.4e6
+    m = c["memory_join"]
+    return (t**m + memory**m) ** (1 / m) + c["launch"]
+
+
 def rank_fa_configs(configs, arch, shape, causal: bool = False, top_n: int | None = None):
-    """Sort FlashAttention configs by `fa_score` (best first)."""
-    ranked = sorted(configs, key=lambda c: fa_score(c, arch, shape, causal), reverse=True)
+    """Sort FlashAttention configs, best first: by `fa_time` at the head dims it was fitted for
+    (64 and 128), by `fa_score` at others.
+
+    Whether the waves should split the keys (`kv_split`) is the choice where the two models differ
+    most and each knows something: where `fa_score` puts such a form first its time counts 0.88,
+    else 1.06 (mean distance to the best measured form 3.2 % either way without the factors and
+    with them, but choices that were right before stay; with 1.15 one shape is 76 % off)."""
+    if shape[4] in (64, 128):
+        whole = [c for c in configs if not getattr(c, "edge", False)]
+        split_first = whole and max(whole, key=lambda c: fa_score(c, arch, shape, causal)).kv_split
+        factor = 0.88 if split_first else 1.06
+        ranked = sorted(configs, key=lambda c: fa_time(c, arch, shape, causal) * (factor if c.kv_split else 1.0))
+    else:
+        ranked = sorted(configs, key=lambda c: fa_score(c, arch, shape, causal), reverse=True)
     return ranked[:top_n] if top_n else ranked

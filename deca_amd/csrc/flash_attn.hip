@@ -29,6 +29,14 @@
 //                       eight; S_q = S_kv = 512, D 64, causal: 9.9 and 5.2 us).  Bound
 //                       then: the CU's load path, which streams all K/V of a row (4 MiB at
 //                       64 B/clk: 28 us of the 49).
+//   DECA_QEDGE          1: the workgroups' query rows need not divide the sequence: the last one's
+//                       reach beyond it, with clamped loads and masked stores, and a wave all of
+//                       whose rows do computes nothing (plain loops).  A sequence that is an odd
+//                       multiple of 64 otherwise only has workgroups of 64 rows and two waves,
+//                       which each pull all of K and V through their CU's load path: B4 H8 S 3392
+//                       D 64 135 us in the best of them, 106 us with 256 rows (the last tile a
+//                       quarter full); B9 H16 S 576 D 128 causal 1.4x.  Bound then as the other
+//                       forms of the tile are, less the rows computed for nothing.
 //   DECA_CAUSAL         1: key j visible to query i iff j <= i (SQ == SKV)
 //   DECA_SCALE          softmax scale
 //   DECA_PIPE           1: S^T of the next tile is computed before the softmax of
@@ -104,6 +112,9 @@
 #ifndef DECA_KVSPLIT
 #define DECA_KVSPLIT 0
 #endif
+#ifndef DECA_QEDGE
+#define DECA_QEDGE 0
+#endif
 // In the 16x16x32 form the plain loops take a tile's row sums on the matrix pipe (one more
 // product per k-step, with a ones operand: four accumulator registers per query tile), which
 // frees the vector ALU of one add per score; l is then the sum of the fp16 P that the second
@@ -177,7 +188,8 @@ static_assert(D_ % 64 == 0 && D_ >= 64, "head dim: a multiple of 64 (flash_attn_
 static_assert(WQ % 32 == 0 && BR % WQ == 0, "each wave owns a multiple of 32 query rows");
 static_assert(!DECA_KVSPLIT || (DECA_PIPE == 0 && !DECA_QSMEM && NW >= 2), "key split: plain loop, Q in registers");
 static_assert(BC % 32 == 0, "BC must be a multiple of 32");
-static_assert(DECA_SQ % BR == 0 && DECA_SKV % BC == 0, "tiles must divide the sequences");
+static_assert((DECA_SQ % BR == 0 || DECA_QEDGE) && DECA_SKV % BC == 0, "tiles must divide the sequences");
+static_assert(DECA_SQ % 32 == 0, "a 32-row block of queries lies in the sequence or beyond it");
 static_assert(TILE_CHUNKS % KV_NT == 0, "loader coverage");
 static_assert(STAGES >= 1 && STAGES <= 3, "K/V ring depth");
 static_assert(STAGES < 3 || DECA_PIPE == 0, "three stages: plain loop only");
@@ -338,7 +350,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   // 1-D grid.  Workgroups are dealt round-robin to the 8 XCDs; the remap gives
   // each XCD whole (batch, head) slices, so that the K/V tiles of a slice are
   // fetched into one L2 only and shared there by all of its query tiles.
-  constexpr int NQ = DECA_SQ / BR;
+  constexpr int NQ = (DECA_SQ + BR - 1) / BR;
   constexpr int TOTAL = NQ * DECA_B * DECA_H;
 #if DECA_CAUSAL
   // Query tiles near the end see the most keys.  They are scheduled first
@@ -363,7 +375,8 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     bh = blockIdx.x % BH;
     qt = (NQ - 1) - blockIdx.x / BH;
   }
-  const int nkv_all = ((qt + 1) * BR + BC - 1) / BC;
+  const int nkv_row = ((qt + 1) * BR + BC - 1) / BC;
+  const int nkv_all = DECA_QEDGE ? min(nkv_row, NKV) : nkv_row;
 #else
   int lin = blockIdx.x;
   if (TOTAL % 8 == 0) lin = (lin & 7) * (TOTAL / 8) + (lin >> 3);
@@ -372,6 +385,15 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   const int nkv_all = NKV;
 #endif
   const int nkv = (nkv_all - kvg + KVG - 1) / KVG;  // (a wave's share may be empty)
+  // First row of this wave, and (DECA_QEDGE) how many rows there are from it on: a row beyond the
+  // sequence is loaded as the last one again and not stored.
+  const int q_row0 = qt * BR + qw * WQ;
+  const int q_row0_u = qt * BR + qw_u * WQ;
+  auto q_row = [&](int r) __attribute__((always_inline)) {  // row r of the wave, relative to q_row0
+    return DECA_QEDGE ? min(q_row0 + r, DECA_SQ - 1) - q_row0 : r;
+  };
+  auto q_inside = [&](int r) __attribute__((always_inline)) { return !DECA_QEDGE || q_row0 + r < DECA_SQ; };
+  const bool q_idle = DECA_QEDGE && q_row0_u >= DECA_SQ;  // no row of this wave lies in the sequence
   const _Float16* q_base = Q + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + qw * WQ) * D_;
   const _Float16* k_base = K + static_cast<size_t>(bh) * DECA_SKV * D_ + kvg * (BC * D_);
   const _Float16* v_base = V + static_cast<size_t>(bh) * DECA_SKV * D_ + kvg * (BC * D_);
@@ -452,12 +474,18 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     constexpr int Q_IT = WQ * CPR / 64;
     static_assert((WQ * CPR) % 64 == 0, "a wave's Q rows are whole 1 KiB runs");
     const unsigned dst = lds_u + Q_LDS_OFFSET + wave_u * (WQ * D_ * 2);
+#if DECA_QEDGE
+    const _Float16* q_origin = Q + (static_cast<size_t>(bh) * DECA_SQ + min(q_row0_u, DECA_SQ - 1)) * D_;
+#else
     const _Float16* q_origin = Q + (static_cast<size_t>(bh) * DECA_SQ + qt * BR + qw_u * WQ) * D_;
+#endif
 #pragma unroll
     for (int it = 0; it < Q_IT; ++it) {
       const int sidx = it * 64 + lane;
       const int row = sidx / CPR, cs = sidx % CPR;
-      dma16(q_origin, static_cast<unsigned>(row * D_ + (cs ^ k_swz(row)) * 8) * 2u, dst + it * 1024);
+      // (a row beyond the sequence lies before q_origin where the whole wave does: 32-bit offsets
+      // are unsigned, so the wave's origin is clamped, too)
+      dma16(q_origin, static_cast<unsigned>((DECA_QEDGE ? q_row(row) - q_row(0) : row) * D_ + (cs ^ k_swz(row)) * 8) * 2u, dst + it * 1024);
     }
   }
 #else
@@ -467,7 +495,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
 #pragma unroll
     for (int ks = 0; ks < DK; ++ks)
       qf[mq][ks] = *reinterpret_cast<const half8*>(
-          q_base + (mq * TQ + lq) * D_ + ks * (K_CHUNKS_PER_STEP * 8) + lg * 8);
+          q_base + q_row(mq * TQ + lq) * D_ + ks * (K_CHUNKS_PER_STEP * 8) + lg * 8);
 #endif
 
   acc_t o_acc[DT][MQ];
@@ -832,9 +860,9 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
     // there is nothing to add.  (Skipping single masked 32-key blocks of the
     // diagonal tiles as well was tried: the extra code paths cost registers and
     // made the kernel slower.)
-    const bool skip = key0(j) > qt * BR + qw_u * WQ + WQ - 1;
+    const bool skip = q_idle || key0(j) > qt * BR + qw_u * WQ + WQ - 1;
 #else
-    const bool skip = false;
+    const bool skip = q_idle;
 #endif
     // one burst behind the barrier, or (DECA_SPREAD) dealt over the S^T groups below
     if (more && (SPREAD_N == 0 || skip)) {
@@ -1411,7 +1439,8 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
       half4 h;
 #pragma unroll
       for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(o[e] * inv);
-      *reinterpret_cast<half4*>(o_base + (mq * TQ + lq) * D_ + lg * 4 + dt * TQ + g * 8) = h;
+      if (q_inside(mq * TQ + lq))
+        *reinterpret_cast<half4*>(o_base + (mq * TQ + lq) * D_ + lg * 4 + dt * TQ + g * 8) = h;
     }
   }
 #else
@@ -1446,7 +1475,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
         half4 h;
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(o_acc[dt][mq][g * 4 + e] * inv);
-        *reinterpret_cast<half4*>(o_row + dt * TQ + g * 8) = h;
+        if (EPI_LDS || q_inside(mq * TQ + lq)) *reinterpret_cast<half4*>(o_row + dt * TQ + g * 8) = h;
       }
   }
   if (EPI_LDS) {
@@ -1459,7 +1488,7 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
       const int idx = it * 64 + lane;
       const int row = idx / CPR, c = idx % CPR;
       const u32x4 v = *reinterpret_cast<const u32x4*>(o_lds + row * EPI_LD + c * 8);
-      *reinterpret_cast<u32x4*>(o_base + row * D_ + c * 8) = v;
+      if (q_inside(row)) *reinterpret_cast<u32x4*>(o_base + row * D_ + c * 8) = v;
     }
   }
 #endif  // DECA_KVSPLIT

@@ -76,6 +76,9 @@ class FAConfig:
     # maxima, sums and O^T meet in LDS at the end.  For grids with too few query rows to give
     # every SIMD a wave of its own.
     kv_split: bool = False
+    # The workgroups' query rows need not divide S_q: the last workgroup of a (batch, head) slice
+    # reaches beyond it, with clamped loads and masked stores.
+    edge: bool = False
 
     @property
     def wave_rows(self) -> int:
@@ -99,7 +102,13 @@ class FAConfig:
             + (f",spread={self.spread}" if self.spread else "")
             + (",trust=1" if self.trust else "")
             + (",kvs=1" if self.kv_split else "")
+            + (",edge=1" if self.edge else "")
         )
+
+
+def query_tiles(cfg: FAConfig, S_q: int) -> int:
+    """Workgroups per (batch, head) slice."""
+    return -(-S_q // cfg.Br)
 
 
 def default_spread(cfg: FAConfig) -> int:
@@ -208,7 +217,9 @@ def check_config(cfg: FAConfig, S_q: int, S_kv: int, D: int) -> None:
     assert not cfg.kv_split or (int(cfg.pipe) == 0 and not cfg.q_in_smem and cfg.num_warps >= 2), \
         "the key split is a form of the plain loop with Q in registers"
     assert cfg.Bc % 32 == 0
-    assert S_q % cfg.Br == 0 and S_kv % cfg.Bc == 0
+    assert S_kv % cfg.Bc == 0
+    # (a wave's 32-row blocks of queries lie in the sequence or beyond it)
+    assert S_q % cfg.Br == 0 or (cfg.edge and S_q % 32 == 0)
     cpr = D // 8
     loaders = WAVE if cfg.kv_split else cfg.threads  # lanes that bring in one K/V tile
     assert (cfg.Bc * cpr) % loaders == 0
@@ -272,12 +283,14 @@ def make_flash_attn_fwd(
         defines["DECA_TRUST"] = 1
     if cfg.kv_split:
         defines["DECA_KVSPLIT"] = 1
+    if cfg.edge:
+        defines["DECA_QEDGE"] = 1
     # The three-stage ring, and the one-stage ring of a wave's own (`kv_split`), wait for part
     # of their outstanding loads, which is only right
     # while the tile loads are the loop's only vector-memory traffic: a build that spills
     # (scratch stores share the counter and retire out of order) is refused at load time.
     return make_spec(
-        TEMPLATE, defines, grid=((S_q // cfg.Br) * B * H, 1, 1), block=(cfg.threads, 1, 1), nargs=4,
+        TEMPLATE, defines, grid=(query_tiles(cfg, S_q) * B * H, 1, 1), block=(cfg.threads, 1, 1), nargs=4,
         options=FAST_MATH_OPTIONS,
         meta={"cfg": str(cfg), "causal": causal, "no_scratch": cfg.stages > 2 or (cfg.kv_split and cfg.stages == 1)},
     )

@@ -371,9 +371,29 @@ FA_FULL = [
 ]
 
 
+# Query tiles that reach over the end of the sequence: a block of 32 rows inside and beyond it,
+# waves without a row of their own, a sequence shorter than the tile; every loop, Q in registers
+# and in LDS, stores through LDS and straight from the registers.
+FA_EDGE_CASES = [
+    (1, 2, 160, 256, 64, False, FAConfig(128, 64, 4, 2, edge=True)),
+    (1, 3, 320, 320, 64, True, FAConfig(128, 64, 4, 2, mfma=16, trust=True, edge=True)),
+    (2, 4, 448, 448, 128, True, FAConfig(256, 64, 8, 2, mfma=16, edge=True)),
+    (1, 2, 64, 192, 128, False, FAConfig(128, 64, 4, 2, pipe=2, spread=8, edge=True)),
+    (1, 2, 320, 320, 128, True, FAConfig(128, 64, 4, 2, pipe=2, mfma=16, spread=8, edge=True)),
+    (2, 2, 192, 128, 128, False, FAConfig(128, 32, 4, 3, mfma=16, trust=True, edge=True)),
+    (1, 2, 352, 352, 64, True, FAConfig(256, 32, 4, 3, q_in_smem=True, edge=True)),
+    (1, 8, 288, 160, 64, False, FAConfig(256, 32, 4, 2, q_in_smem=True, mfma=16, roll=True, trust=True, edge=True)),
+    (1, 2, 96, 96, 128, True, FAConfig(128, 32, 4, 1, mfma=16, edge=True)),
+    (1, 1, 416, 128, 64, False, FAConfig(256, 128, 8, 1, edge=True)),
+    (1, 2, 192, 192, 192, True, FAConfig(128, 64, 4, 2, spread=4, edge=True)),
+    (1, 2, 96, 128, 64, False, FAConfig(64, 32, 4, 1, kv_split=True, edge=True)),
+    (1, 2, 352, 128, 128, False, FAConfig(256, 64, 8, 2, pipe=1, edge=True)),
+]
+
+
 def fa_specs():
     return [make_flash_attn_fwd(B, H, Sq, Skv, D, cfg, None, causal)
-            for B, H, Sq, Skv, D, causal, cfg in FA_CASES + FA_SPLIT_CASES + FA_FULL]
+            for B, H, Sq, Skv, D, causal, cfg in FA_CASES + FA_SPLIT_CASES + FA_EDGE_CASES + FA_FULL]
 
 
 def spilling_specs():
