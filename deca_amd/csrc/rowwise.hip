@@ -22,6 +22,8 @@
 //                3001 x 5124: 14.3 us with 8-byte accesses and 128 lanes a row, 11.4 us with
 //                these and a wave a row (3001 x 5120, whose rows are aligned: 10.6); softmax
 //                bf16 777 x 65532: 52.0 and 45.9 us
+//   DECA_ONLINE  1 (reg mode, VEC = 8, whole waves a row): the first pass takes the chunks of a
+//                row as they arrive (see there)
 //   DECA_EPS     RMSNorm epsilon
 //
 // Lane t of a row owns the VEC-element chunks (c * TPR + t) * VEC, so one wave
@@ -75,6 +77,11 @@ typedef vec_t mem_t;
 #ifndef DECA_LEAN
 #define DECA_LEAN 0
 #endif
+#ifndef DECA_ONLINE
+#define DECA_ONLINE 0
+#endif
+static_assert(!DECA_ONLINE || (DECA_MODE == 0 && VEC == 8 && TPR % 64 == 0),
+              "online: reg mode, 16-byte accesses, whole waves a row");
 
 #define LOG2E 1.4426950408889634f
 #define NEG_INF (-1e30f)
@@ -218,7 +225,133 @@ deca_main(const elem_t* __restrict__ x,
   auto store_row = [&](int c, vec_t v) { store_vec(yr + col(c), v); };
 #endif
 
-#if DECA_MODE == 0
+#if DECA_ONLINE
+  // ------------------------- reg mode, chunks as they arrive -------------------------
+  // Softmax: exponentials against the lane's max so far, whose sum is rescaled when that grows,
+  // so that behind the last chunk only the reduction is left, of max and sum in one exchange.  A
+  // row whose workgroup has a CU (nearly) to itself otherwise adds two passes of vector work over
+  // the row to the time of its loads and stores, with the memory idle (bf16, 1024 lanes a row:
+  // 1024 x 128256 105.6 -> 96.4 us, 5.45 TB/s; 2020 x 63956 99.1 -> 94.6; 275 x 118396 41.7 -> 34.8).
+  // Bound then: the last exchange, the exponentials of the stores and the next workgroup's start,
+  // which other rows of the CU only hide in part (a copy of the same size runs at 6.4 TB/s).
+  // All accesses go through a buffer descriptor of the row: one lane offset and a constant per
+  // chunk instead of 64-bit addresses, and the range check leaves out what the last chunk has beyond
+  // the end (its offset is all in the lane's own address, which is what is checked).
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  constexpr int AUX = DECA_HINT ? 2 : 0;  // non-temporal
+  const int rbu = __builtin_amdgcn_readfirstlane(rb);
+  const unsigned lane_off = t * (VEC * 2);
+  const unsigned tail_off = lane_off + C_FULL * (SPAN * 2);
+  auto row_of = [&](const elem_t* base) {
+    const elem_t* p = base + (static_cast<size_t>(blockIdx.x) * RPB + rbu) * DECA_N;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<elem_t*>(p), 0, DECA_N * 2, 0x00027000);
+  };
+  const auto src = row_of(x), dst = row_of(y);
+  // (the last vector of a row may be a half: two accesses, each in the row or not)
+  vec_t xh[NCHUNK];
+#pragma unroll
+  for (int c = 0; c < NCHUNK; ++c) {
+    if (c < C_FULL) {
+      xh[c] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(src, lane_off, c * (SPAN * 2), AUX));
+    } else if (DECA_HALF) {
+      const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(src, tail_off, 0, AUX);
+      const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(src, tail_off + 8, 0, AUX);
+      const u32x4 both = {lo.x, lo.y, hi.x, hi.y};
+      xh[c] = __builtin_bit_cast(vec_t, both);
+    } else {
+      xh[c] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(src, tail_off, 0, AUX));
+    }
+  }
+  // (all requests first: the scheduler would put off the later ones until the first pass is under
+  // way, 91.5 -> 93.6 us for 2048 x 65536 bf16)
+  __builtin_amdgcn_sched_barrier(0);
+  // (stores carry all of their offset in the lane's address: after one with an offset in a scalar
+  // register the compiler leaves out the wait that its data needs before they are overwritten)
+  auto put = [&](int c, vec_t v) {
+    const u32x4 u = __builtin_bit_cast(u32x4, v);
+    if (c < C_FULL) {
+      __builtin_amdgcn_raw_buffer_store_b128(u, dst, lane_off + c * (SPAN * 2), 0, AUX);
+    } else if (DECA_HALF) {
+      const u32x2 lo = {u.x, u.y}, hi = {u.z, u.w};
+      __builtin_amdgcn_raw_buffer_store_b64(lo, dst, tail_off, 0, AUX);
+      __builtin_amdgcn_raw_buffer_store_b64(hi, dst, tail_off + 8, 0, AUX);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b128(u, dst, tail_off, 0, AUX);
+    }
+  };
+  static_assert(DECA_OP == 0, "online: softmax");
+  // The sums are rescaled by the difference of the rounded products max * log2(e) that the
+  // exponents were formed with, not of the maxima: as in the two-pass form, that rounding then
+  // cancels in the quotient, however large the elements are.  Beyond 1e9 it makes exponentials of
+  // the largest elements themselves infinite, and a lane may hold no other ones (masked by a large
+  // negative number): held finite, so that the rescale makes them 0 and not NaN.  (Opaque to the
+  // optimiser, which would put the product back into the exponents and knows no infinities.)
+  auto scaled = [&](float v) __attribute__((always_inline)) {
+    float p = v * LOG2E;
+    asm volatile("" : "+v"(p));
+    return p;
+  };
+  auto finite = [&](float v) __attribute__((always_inline)) {
+    unsigned u = __builtin_bit_cast(unsigned, v);
+    asm volatile("" : "+v"(u));
+    return __builtin_bit_cast(float, u == 0x7f800000u ? 0x7f7fffffu : u);
+  };
+  float m = NEG_INF, m2 = NEG_INF * LOG2E, sum = 0.0f;
+  constexpr int AT_ONCE = 2;  // chunks per rescale of the sum
+#pragma unroll
+  for (int c0 = 0; c0 < NCHUNK; c0 += AT_ONCE) {
+#pragma unroll
+    for (int c = c0; c < c0 + AT_ONCE && c < NCHUNK; ++c)
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) m = fmaxf(m, elem_ok(c, i) ? static_cast<float>(xh[c][i]) : NEG_INF);
+    const float before = m2;
+    m2 = scaled(m);
+    float acc = 0.0f;
+#pragma unroll
+    for (int c = c0; c < c0 + AT_ONCE && c < NCHUNK; ++c)
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) {
+        const float v = elem_ok(c, i) ? static_cast<float>(xh[c][i]) : NEG_INF;
+        acc += fast_exp2(v * LOG2E - m2);
+      }
+    sum = finite(sum * fast_exp2(before - m2) + acc);
+  }
+  const float top2 = wave_allreduce<RED_LANES>(m2, MaxOp());
+  sum = wave_allreduce<RED_LANES>(sum * fast_exp2(m2 - top2), AddOp());
+  m2 = top2;
+#if NW > 1
+  float* tops = red0 + rb * NW;
+  float* sums = red1 + rb * NW;
+  if (lane == 0) {
+    tops[wr] = m2;
+    sums[wr] = finite(sum);
+  }
+  __syncthreads();
+  float tops2[NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    tops2[i] = tops[i];
+    m2 = fmaxf(m2, tops2[i]);
+  }
+  sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) sum += sums[i] * fast_exp2(tops2[i] - m2);
+#endif
+  const float inv = __builtin_amdgcn_rcpf(sum);
+  // (nothing but the packed row is kept from the first pass)
+#pragma unroll
+  for (int c = 0; c < NCHUNK; ++c) asm volatile("" : "+v"(xh[c]));
+#pragma unroll
+  for (int c = 0; c < NCHUNK; ++c) {
+    vec_t o;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      o[i] = static_cast<elem_t>(fast_exp2(static_cast<float>(xh[c][i]) * LOG2E - m2) * inv);
+    put(c, o);
+  }
+
+#elif DECA_MODE == 0
   // ------------------------------ reg mode ------------------------------
   vec_t xh[NCHUNK];
 #pragma unroll

@@ -111,8 +111,33 @@ def use_lean(cfg: RowConfig, N: int, op: str) -> bool:
             and _fits(lean_regs_per_thread(cfg, N), cfg.threads))
 
 
+# Softmax rows from this length on take their first pass as the chunks arrive, in workgroups of 512
+# lanes a row or more.  Measured against the two-pass form of the same lanes: 1.00-1.20x on 91 of 94
+# kernels of 47 shapes from 51.5K to 129K elements, behind by at most 1.5 % on the others (1024 x
+# 128256 bf16 106 -> 96 us, 538 x 53396 fp16 30 -> 25, 275 x 118396 bf16 42 -> 35); level with it from
+# 34K to 50K, 2-18 % behind on shorter rows, whose CUs hold other rows to fill the gaps, and level
+# with it for 256 lanes.
+ONLINE_MIN_N = 50000
+ONLINE_MIN_TPR = 512
+
+
+def online_regs_per_thread(cfg: RowConfig, N: int) -> int:
+    """Estimate for the online form: the packed row and what two chunks are worked on with
+    (VGPRs measured: 59 at 8 chunks a lane, 88-93 at 16, 152 at 32)."""
+    return num_chunks(cfg, N) * 4 + 30
+
+
+def use_online(cfg: RowConfig, N: int, op: str) -> bool:
+    """Whether a config is compiled in its online form."""
+    return (op == "softmax" and cfg.mode == "reg" and cfg.vec == 8 and N >= ONLINE_MIN_N
+            and cfg.threads_per_row >= ONLINE_MIN_TPR
+            and _fits(online_regs_per_thread(cfg, N), cfg.threads))
+
+
 def regs_per_thread(cfg: RowConfig, N: int, op: str) -> int:
-    """Estimate of the form that gets compiled (plain or lean)."""
+    """Estimate of the form that gets compiled (plain, lean or online)."""
+    if use_online(cfg, N, op):
+        return online_regs_per_thread(cfg, N)
     return lean_regs_per_thread(cfg, N) if use_lean(cfg, N, op) else est_regs_per_thread(cfg, N, op)
 
 
@@ -161,6 +186,8 @@ def make_rowwise(
     }
     if use_lean(cfg, N, op):
         defines["DECA_LEAN"] = 1
+    if use_online(cfg, N, op):  # (which keeps no more than the lean form does)
+        defines["DECA_ONLINE"] = 1
     if cfg.half:
         defines["DECA_HALF"] = 1
     return make_spec(

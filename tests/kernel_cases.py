@@ -58,6 +58,23 @@ ROWWISE_CASES = [
     ("rmsnorm", 7, 128260, "float16", RowConfig(512, 1, 8, half=True)),
 ]
 
+# Softmax rows whose first pass takes the chunks as they arrive: the shortest such row, whole and
+# half last vectors, chunks that end with the row and not, odd numbers of chunks, the longest rows
+# of the registers, several rows per workgroup, plain and hinted
+ROWWISE_ONLINE_CASES = [
+    ("softmax", 6, 50000, "float16", RowConfig(512, 1, 8, hint=True)),
+    ("softmax", 6, 50004, "bfloat16", RowConfig(512, 1, 8, hint=True, half=True)),
+    ("softmax", 6, 50008, "float16", RowConfig(1024, 1, 8)),
+    ("softmax", 6, 57348, "float16", RowConfig(512, 2, 8, half=True)),
+    ("softmax", 6, 65536, "bfloat16", RowConfig(512, 1, 8)),
+    ("softmax", 6, 65536, "float16", RowConfig(1024, 1, 8, hint=True)),
+    ("softmax", 6, 73732, "bfloat16", RowConfig(1024, 1, 8, half=True)),
+    ("softmax", 6, 128252, "float16", RowConfig(1024, 1, 8, hint=True, half=True)),
+    ("softmax", 6, 128256, "bfloat16", RowConfig(1024, 1, 8, hint=True)),
+    ("softmax", 6, 131072, "bfloat16", RowConfig(512, 1, 8, hint=True)),
+    ("softmax", 6, 131072, "float16", RowConfig(1024, 1, 8, hint=True)),
+]
+
 # Full-size benchmark shapes (property checks + a sampled comparison).
 ROWWISE_FULL = [
     ("softmax", 16384, 4096, "float16", RowConfig(128, 1, 8)),
@@ -67,7 +84,8 @@ ROWWISE_FULL = [
 
 
 def rowwise_specs(eps: float = 1e-6):
-    return [make_rowwise(op, M, N, dt, cfg, eps) for op, M, N, dt, cfg in ROWWISE_CASES + ROWWISE_FULL]
+    return [make_rowwise(op, M, N, dt, cfg, eps)
+            for op, M, N, dt, cfg in ROWWISE_CASES + ROWWISE_ONLINE_CASES + ROWWISE_FULL]
 
 
 # (M, N, K, cfg): sizes the CPU checker finishes in seconds
