@@ -120,6 +120,28 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
 
     tail = N / (chunks * cfg.threads_per_row * cfg.vec) if cfg.mode == "reg" else 1.0
     lanes = 1.0 if cfg.vec * type_size >= 16 else 0.985
+    # Rows of an odd multiple of 8 bytes have forms with 16-byte accesses (`half`).  Level with 8-byte
+    # ones in small grids.  With 42 (softmax: 52) to 75 KiB per CU 1.00-1.32x on 37 of 39 shapes of 770
+    # to 18K elements (RMSNorm bf16 1822 x 4628: 9.4 and 7.1 us), 1 % behind on two.  Beyond that
+    # 1.02-1.26x on 49 of 49 from these lengths on, but 1-3 % behind on shorter RMSNorm rows, and 2-11 %
+    # on 7 of 7 of the length where they come to a few chunks of few lanes.
+    if N % 8 == 4 and lanes < 1.0:
+        softmax = op == "softmax"
+        if kib_per_cu <= 75:
+            ahead = kib_per_cu >= (52 if softmax else 42) and N >= 700
+        else:
+            ahead = N >= (4100 if softmax else 3400) and not (5200 if softmax else 6900) < N < 7900
+        if ahead:
+            lanes = 0.93
+    # A workgroup that has a long row to itself leaves a CU room for two or three others, one with
+    # two such rows for none (36K ... 55K elements: 10-37 % behind one row of 256 lanes on 13 of 13
+    # shapes), nor do 1024 lanes (33K ... 50K: 2-42 % behind on 20 of 20; with up to 4.5 rows per CU
+    # 4-42 % on 24 of 26 from 8.6K to 21K).
+    if cfg.rows_per_block > 1 and N > 32768:
+        rows *= 0.85
+    if not online:
+        if cfg.threads_per_row == 1024 and (33000 < N < 50000 or (rows_per_cu <= 4.5 and 8600 < N < 21000)):
+            drain *= 0.88
     stream = 1.0 if cfg.hint else getattr(arch, "rowwise_no_hint_factor", 0.92)
 
     return (mem * granularity * wave_eff * drain * rows * reduce * (0.7 + 0.3 * tail) * lanes *
