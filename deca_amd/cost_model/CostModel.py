@@ -63,24 +63,24 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     - non-temporal accesses: streamed data does not displace lines in L2 /
       Infinity Cache and the writes drain earlier (measured: ~8% on MI355X)
     """
-    from deca_amd.kernels.rowwise_hip import num_chunks, use_online
+    from deca_amd.kernels.rowwise_hip import num_chunks, use_lines, use_online
 
     wgs = rowwise_occupancy(cfg, arch, op, N)
     chunks = num_chunks(cfg, N)
     depth = chunks if cfg.mode == "reg" else cfg.unroll
     grid = M // cfg.rows_per_block
-    # One wave a row with every row resident at once: all loads are under way from the start, no
-    # round waits for another and no waves meet.  Measured against the choice without this term
-    # (60 shapes): RMSNorm 1.02-1.26x from 7 to 16 rows and 96 to 144 KiB per CU (3977 x 4992
-    # at 151 KiB still, nothing from 17 rows on: 5086 x 3464 0.96x); softmax, whose wave has
-    # twice the arithmetic per row to do alone, 1.02-1.26x up to 128 KiB and 0.95-1.02x beyond.
-    # Below 7 rows or 96 KiB (600 x 16384, 512 x 50004, 2048 x 4096) wider rows are 4-50 % ahead.
+    # Every row resident at once: all loads are under way from the start and no round waits for
+    # another.  What counts then is the CU with the most rows and the number of waves on a CU: nine to
+    # twelve, with 64 lanes a row or more as that takes (1341 x 10744: 10.5 us with 5 waves a CU, 10.6
+    # with 10, 11.5 with 21, 11.9 with 42; 780 x 14432: 9.8, 9.0, 8.8 and 10.1 with 3, 6, 12 and 24; more
+    # waves meet in a reduction, fewer leave a SIMD idle).  59 shapes of 45 to 300 KiB per CU: mean
+    # distance to the best 2.3 % (2.9 % in the caches) against 5.2 and 7.4 % by the terms below; longer
+    # softmax rows, whose waves have twice the arithmetic of RMSNorm, gain nothing beyond 140 KiB.
     rows_per_cu = M / arch.sm_nums
     kib_per_cu = rows_per_cu * N * type_size / 1024
-    one_round = (cfg.mode == "reg" and cfg.threads_per_row == arch.warp_size
-                 and cfg.rows_per_block == 1 and cfg.vec * type_size >= 16 and depth <= 16
-                 and grid <= arch.sm_nums * wgs and 7 <= rows_per_cu <= 16
-                 and 96 <= kib_per_cu <= (128 if op == "softmax" else 144))
+    one_round = (cfg.mode == "reg" and cfg.threads_per_row >= arch.warp_size
+                 and cfg.vec * type_size >= 16 and depth <= 20 and grid <= arch.sm_nums * wgs
+                 and 45 <= kib_per_cu <= (140 if op == "softmax" else 210))
     if one_round:
         wgs = max(1, math.ceil(grid / arch.sm_nums))
     in_flight = wgs * cfg.threads * depth * cfg.vec * type_size
@@ -107,7 +107,15 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     if cfg.threads_per_row < arch.warp_size:
         reduce *= 0.97
     if one_round:
-        wave_eff = granularity = 1.0
+        granularity = drain = 1.0
+        wave_eff = math.sqrt(rows_per_cu / (math.ceil(grid / arch.sm_nums) * cfg.rows_per_block))
+        rows = 1.0 / (1.0 + 0.015 * math.log2(cfg.rows_per_block))
+        waves_per_cu = rows_per_cu * waves_per_row
+        reduce = 1.0 / (1.0 + 0.07 * abs(math.log2(waves_per_cu / 10.5)))
+        if cfg.half and waves_per_row == 1 and use_lines(cfg, M, N, op):
+            # both ends of the row are the one wave's to patch (RMSNorm fp16 3001 x 5124: 10.5 us, and
+            # 9.9 with two waves)
+            reduce *= 0.9
     online = use_online(cfg, N, op)
     if online:
         # The first pass is done when the last chunk arrives: what lengthens the others' series of

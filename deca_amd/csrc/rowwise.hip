@@ -24,6 +24,12 @@
 //                bf16 777 x 65532: 52.0 and 45.9 us
 //   DECA_ONLINE  1 (reg mode, VEC = 8, whole waves a row): the first pass takes the chunks of a
 //                row as they arrive (see there)
+//   DECA_LINES   1 (reg mode, VEC = 8, whole waves a row): the lanes' chunks start at the memory line
+//                that the row starts in, so that a wave's accesses are whole lines however the rows
+//                lie.  Rows off the lines had every wave touch one more and share it with the next,
+//                for 3-12 % of the time: softmax bf16 2048 x 84936 135 us (5.15 TB/s) -> 124, where
+//                84992 takes 123; RMSNorm bf16 3001 x 5128 12.3 -> 10.8, 16384 x 4104 46.3 -> 44.6.
+//                The weight is read across lines instead, which the L1 serves.
 //   DECA_EPS     RMSNorm epsilon
 //
 // Lane t of a row owns the VEC-element chunks (c * TPR + t) * VEC, so one wave
@@ -42,19 +48,25 @@
 #error "rowwise.hip is a template: define the DECA_* macros"
 #endif
 
+#ifndef DECA_HALF
+#define DECA_HALF 0
+#endif
 #define TPR DECA_TPR
 #define RPB DECA_RPB
 #define VEC DECA_VEC
 #define NT (TPR * RPB)
 #define SPAN (TPR * VEC)
-#define NCHUNK ((DECA_N + SPAN - 1) / SPAN)
+#ifndef DECA_LINES
+#define DECA_LINES 0
+#endif
+#define LINE 128  // bytes
+// elements by which a row may start behind its line
+#define LINE_PAD (DECA_LINES ? (DECA_HALF ? 60 : 56) : 0)
+#define NCHUNK ((DECA_N + LINE_PAD + SPAN - 1) / SPAN)
 #define C_FULL (DECA_N / SPAN)
 #define RED_LANES (TPR < 64 ? TPR : 64)
 #define NW (TPR / 64 > 0 ? TPR / 64 : 1)
 
-#ifndef DECA_HALF
-#define DECA_HALF 0
-#endif
 static_assert(DECA_HALF ? (VEC == 8 && DECA_N % 8 == 4 && DECA_MODE == 0) : DECA_N % VEC == 0,
               "N must be a multiple of the vector width, or of half of it (DECA_HALF)");
 static_assert(DECA_M % RPB == 0, "M must be a multiple of rows_per_block");
@@ -80,8 +92,11 @@ typedef vec_t mem_t;
 #ifndef DECA_ONLINE
 #define DECA_ONLINE 0
 #endif
-static_assert(!DECA_ONLINE || (DECA_MODE == 0 && VEC == 8 && TPR % 64 == 0),
-              "online: reg mode, 16-byte accesses, whole waves a row");
+// Rows are read and written through a buffer descriptor
+#define BUFFER (DECA_ONLINE || DECA_LINES)
+static_assert(!BUFFER || (DECA_MODE == 0 && VEC == 8 && TPR % 64 == 0),
+              "online, lines: reg mode, 16-byte accesses, whole waves a row");
+static_assert(!DECA_ONLINE || DECA_OP == 0, "online: softmax");
 
 #define LOG2E 1.4426950408889634f
 #define NEG_INF (-1e30f)
@@ -172,6 +187,11 @@ __device__ __forceinline__ void store_vec(elem_t* p, vec_t v) {
 
 __device__ __forceinline__ float fast_exp2(float v) { return __builtin_amdgcn_exp2f(v); }
 
+template <int AUX>
+struct aux_t {
+  static constexpr int value = AUX;
+};
+
 // ---------------------------------------------------------------------------
 // kernel
 // ---------------------------------------------------------------------------
@@ -198,6 +218,127 @@ deca_main(const elem_t* __restrict__ x,
   const elem_t* xr = x + row_base;
   elem_t* yr = y + row_base;
 
+#if BUFFER
+  // All accesses go through a buffer descriptor of the row: a lane offset and a constant per chunk
+  // instead of 64-bit addresses, and the range check takes the place of branches: what lies before
+  // (offsets that wrap) or behind the row is read as 0 and not written.
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  constexpr int AUX = DECA_HINT ? 2 : 0;  // non-temporal
+  const size_t row_u = (static_cast<size_t>(blockIdx.x) * RPB + __builtin_amdgcn_readfirstlane(rb)) * DECA_N;
+  auto row_of = [&](const elem_t* p) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<elem_t*>(p), 0, DECA_N * 2, 0x00027000);
+  };
+  const auto src = row_of(x + row_u), dst = row_of(y + row_u);
+#if DECA_LINES
+  // Bytes of the first line before the row, a multiple of a vector (or of a half one), so that only
+  // rows of an odd number of halves have vectors that reach over an end.
+  const unsigned skip = static_cast<unsigned>(reinterpret_cast<size_t>(x + row_u)) & (LINE - (DECA_HALF ? 8 : 16));
+  constexpr int C_FIRST = 1;
+#else
+  constexpr unsigned skip = 0;
+  constexpr int C_FIRST = 0;
+#endif
+  // chunks that lie in the row for every lane
+  auto inner = [&](int c) __attribute__((always_inline)) { return c >= C_FIRST && c < C_FULL; };
+  const unsigned lane_off = t * (VEC * 2) - skip;
+  const unsigned inner_off = lane_off + C_FIRST * (SPAN * 2);
+  const unsigned wave_off = __builtin_amdgcn_readfirstlane(wr) * (64 * VEC * 2) - skip;
+  // Offset of a vector of a chunk at an end of the row.  (Opaque: the sum must wrap in the register
+  // and not be split into the instruction's own offset.)
+  auto end_off = [&](int c) __attribute__((always_inline)) {
+    unsigned off = lane_off + c * (SPAN * 2);
+    asm volatile("" : "+v"(off));
+    return off;
+  };
+  // The vectors that reach over an end of the row (DECA_HALF): the half inside is accessed by itself.
+  constexpr unsigned NOWHERE = 0xfffffff0u, LAST_HALF = DECA_N * 2u - 8u;
+  auto over_start = [&](int c) __attribute__((always_inline)) {
+    return DECA_HALF && DECA_LINES && c == 0 && lane_off == 0u - 8u;
+  };
+  auto over_end = [&](int c) __attribute__((always_inline)) {
+    return DECA_HALF && c >= C_FULL && lane_off + c * (SPAN * 2) == LAST_HALF;
+  };
+  struct ends_t {
+    u32x2 start, end;
+  };
+  auto ends_of = [&](auto rsrc, auto aux) __attribute__((always_inline)) {
+    ends_t e = {};
+#if DECA_HALF
+    // (by all lanes of the waves that hold an end: a branch of some lanes would wait for the others)
+    constexpr int HINT = decltype(aux)::value;
+    if (DECA_LINES && wave_off == 0u - skip)
+      e.start = __builtin_amdgcn_raw_buffer_load_b64(rsrc, over_start(0) ? 0u : NOWHERE, 0, HINT);
+    bool lane_end = false, wave_end = false;
+#pragma unroll
+    for (int c = C_FULL; c < NCHUNK; ++c) {
+      lane_end |= over_end(c);
+      wave_end |= LAST_HALF - (wave_off + c * (SPAN * 2)) < 64u * VEC * 2;
+    }
+    if (wave_end) e.end = __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane_end ? LAST_HALF : NOWHERE, 0, HINT);
+#endif
+    return e;
+  };
+  auto elem_ok = [&](int c, int i) __attribute__((always_inline)) {
+    return inner(c) || lane_off + c * (SPAN * 2) + (DECA_HALF && i >= 4 ? 8 : 0) < DECA_N * 2u;
+  };
+  auto fetch = [&](auto rsrc, int c, auto aux) __attribute__((always_inline)) {
+    constexpr int HINT = decltype(aux)::value;
+    if (inner(c))
+      return __builtin_bit_cast(
+          vec_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, inner_off, (c - C_FIRST) * (SPAN * 2), HINT));
+    const unsigned off = end_off(c);
+    return __builtin_bit_cast(
+        vec_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, over_end(c) ? NOWHERE : off, 0, HINT));
+  };
+  auto join = [&](vec_t x, const ends_t& e, int c) __attribute__((always_inline)) {
+    u32x4 v = __builtin_bit_cast(u32x4, x);
+    if (over_start(c)) v = u32x4{0, 0, e.start.x, e.start.y};
+    if (over_end(c)) v = u32x4{e.end.x, e.end.y, 0, 0};
+    return __builtin_bit_cast(vec_t, v);
+  };
+  // (of a wave: whether any of its lanes holds elements of the chunk)
+  auto in_row = [&](int c) __attribute__((always_inline)) {
+    return c < C_FULL || static_cast<int>(wave_off + c * (SPAN * 2)) < DECA_N * 2;
+  };
+  const ends_t x_ends = ends_of(src, aux_t<AUX>());
+  auto load_x = [&](int c) __attribute__((always_inline)) { return fetch(src, c, aux_t<AUX>()); };
+  // (behind all loads: what has to wait for one ends where another is conditional)
+  auto join_x = [&](vec_t(&row)[NCHUNK]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < NCHUNK; ++c) row[c] = join(row[c], x_ends, c);
+  };
+#if DECA_OP == 1
+  const auto weights = row_of(w);  // (as long as a row)
+  const ends_t w_ends = ends_of(weights, aux_t<0>());
+  auto load_w = [&](const elem_t*, int c) __attribute__((always_inline)) {
+    return join(fetch(weights, c, aux_t<0>()), w_ends, c);
+  };
+#endif
+  // (Stores carry all of their offset in the lane's address: after one with an offset in a scalar
+  // register the compiler leaves out the wait that its data needs before they are overwritten.)
+  ends_t y_ends = {};
+  auto store_row = [&](int c, vec_t v) __attribute__((always_inline)) {
+    const u32x4 u = __builtin_bit_cast(u32x4, v);
+    if (inner(c)) {
+      __builtin_amdgcn_raw_buffer_store_b128(u, dst, inner_off + (c - C_FIRST) * (SPAN * 2), 0, AUX);
+      return;
+    }
+    const unsigned off = end_off(c);
+    __builtin_amdgcn_raw_buffer_store_b128(u, dst, over_end(c) ? NOWHERE : off, 0, AUX);
+    if (DECA_LINES && c == 0) y_ends.start = u32x2{u.z, u.w};
+    if (over_end(c)) y_ends.end = u32x2{u.x, u.y};
+  };
+  auto store_ends = [&]() __attribute__((always_inline)) {
+#if DECA_HALF
+    if (over_start(0)) __builtin_amdgcn_raw_buffer_store_b64(y_ends.start, dst, 0, 0, AUX);
+    bool lane_end = false;
+#pragma unroll
+    for (int c = C_FULL; c < NCHUNK; ++c) lane_end |= over_end(c);
+    if (lane_end) __builtin_amdgcn_raw_buffer_store_b64(y_ends.end, dst, LAST_HALF, 0, AUX);
+#endif
+  };
+#else
   auto col = [&](int c) { return (c * TPR + t) * VEC; };
   // Chunks >= C_FULL are out of the row for the upper lanes.
   auto in_row = [&](int c) { return c < C_FULL || col(c) < DECA_N; };
@@ -225,6 +366,8 @@ deca_main(const elem_t* __restrict__ x,
   auto store_row = [&](int c, vec_t v) { store_vec(yr + col(c), v); };
 #endif
 
+#endif  // BUFFER
+
 #if DECA_ONLINE
   // ------------------------- reg mode, chunks as they arrive -------------------------
   // Softmax: exponentials against the lane's max so far, whose sum is rescaled when that grows,
@@ -234,53 +377,13 @@ deca_main(const elem_t* __restrict__ x,
   // 1024 x 128256 105.6 -> 96.4 us, 5.45 TB/s; 2020 x 63956 99.1 -> 94.6; 275 x 118396 41.7 -> 34.8).
   // Bound then: the last exchange, the exponentials of the stores and the next workgroup's start,
   // which other rows of the CU only hide in part (a copy of the same size runs at 6.4 TB/s).
-  // All accesses go through a buffer descriptor of the row: one lane offset and a constant per
-  // chunk instead of 64-bit addresses, and the range check leaves out what the last chunk has beyond
-  // the end (its offset is all in the lane's own address, which is what is checked).
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-  constexpr int AUX = DECA_HINT ? 2 : 0;  // non-temporal
-  const int rbu = __builtin_amdgcn_readfirstlane(rb);
-  const unsigned lane_off = t * (VEC * 2);
-  const unsigned tail_off = lane_off + C_FULL * (SPAN * 2);
-  auto row_of = [&](const elem_t* base) {
-    const elem_t* p = base + (static_cast<size_t>(blockIdx.x) * RPB + rbu) * DECA_N;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<elem_t*>(p), 0, DECA_N * 2, 0x00027000);
-  };
-  const auto src = row_of(x), dst = row_of(y);
-  // (the last vector of a row may be a half: two accesses, each in the row or not)
   vec_t xh[NCHUNK];
 #pragma unroll
-  for (int c = 0; c < NCHUNK; ++c) {
-    if (c < C_FULL) {
-      xh[c] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(src, lane_off, c * (SPAN * 2), AUX));
-    } else if (DECA_HALF) {
-      const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(src, tail_off, 0, AUX);
-      const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(src, tail_off + 8, 0, AUX);
-      const u32x4 both = {lo.x, lo.y, hi.x, hi.y};
-      xh[c] = __builtin_bit_cast(vec_t, both);
-    } else {
-      xh[c] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(src, tail_off, 0, AUX));
-    }
-  }
+  for (int c = 0; c < NCHUNK; ++c) xh[c] = in_row(c) ? load_x(c) : vec_t{};
   // (all requests first: the scheduler would put off the later ones until the first pass is under
   // way, 91.5 -> 93.6 us for 2048 x 65536 bf16)
   __builtin_amdgcn_sched_barrier(0);
-  // (stores carry all of their offset in the lane's address: after one with an offset in a scalar
-  // register the compiler leaves out the wait that its data needs before they are overwritten)
-  auto put = [&](int c, vec_t v) {
-    const u32x4 u = __builtin_bit_cast(u32x4, v);
-    if (c < C_FULL) {
-      __builtin_amdgcn_raw_buffer_store_b128(u, dst, lane_off + c * (SPAN * 2), 0, AUX);
-    } else if (DECA_HALF) {
-      const u32x2 lo = {u.x, u.y}, hi = {u.z, u.w};
-      __builtin_amdgcn_raw_buffer_store_b64(lo, dst, tail_off, 0, AUX);
-      __builtin_amdgcn_raw_buffer_store_b64(hi, dst, tail_off + 8, 0, AUX);
-    } else {
-      __builtin_amdgcn_raw_buffer_store_b128(u, dst, tail_off, 0, AUX);
-    }
-  };
-  static_assert(DECA_OP == 0, "online: softmax");
+  join_x(xh);
   // The sums are rescaled by the difference of the rounded products max * log2(e) that the
   // exponents were formed with, not of the maxima: as in the two-pass form, that rounding then
   // cancels in the quotient, however large the elements are.  Beyond 1e9 it makes exponentials of
@@ -348,8 +451,9 @@ deca_main(const elem_t* __restrict__ x,
 #pragma unroll
     for (int i = 0; i < VEC; ++i)
       o[i] = static_cast<elem_t>(fast_exp2(static_cast<float>(xh[c][i]) * LOG2E - m2) * inv);
-    put(c, o);
+    if (in_row(c)) store_row(c, o);
   }
+  store_ends();
 
 #elif DECA_MODE == 0
   // ------------------------------ reg mode ------------------------------
@@ -357,7 +461,13 @@ deca_main(const elem_t* __restrict__ x,
 #pragma unroll
   for (int c = 0; c < NCHUNK; ++c) {
     if (in_row(c)) xh[c] = load_x(c);
+#if BUFFER
+    else xh[c] = vec_t{};
+#endif
   }
+#if BUFFER
+  join_x(xh);
+#endif
 
 #if DECA_OP == 0
   float m = NEG_INF;
@@ -405,7 +515,8 @@ deca_main(const elem_t* __restrict__ x,
   for (int c = 0; c < NCHUNK; ++c) {
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
-      const float v = elem_ok(c, i) ? static_cast<float>(xh[c][i]) : 0.0f;
+      // (a buffer load beyond the row returns 0)
+      const float v = BUFFER || elem_ok(c, i) ? static_cast<float>(xh[c][i]) : 0.0f;
       ss += v * v;
     }
   }
@@ -429,6 +540,9 @@ deca_main(const elem_t* __restrict__ x,
       store_row(c, o);
     }
   }
+#endif
+#if BUFFER
+  store_ends();
 #endif
 
 #else

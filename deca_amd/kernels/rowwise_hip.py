@@ -134,6 +134,41 @@ def use_online(cfg: RowConfig, N: int, op: str) -> bool:
             and _fits(online_regs_per_thread(cfg, N), cfg.threads))
 
 
+LINE = 128  # bytes of a memory line
+
+
+def use_lines(cfg: RowConfig, M: int, N: int, op: str) -> bool:
+    """Whether the lanes' chunks start at the memory line that the row starts in (rows that are no
+    whole number of lines).
+
+    Measured against chunks that start with the row, on 379 shapes, by KiB of input per CU.  Rows of
+    whole vectors: RMSNorm 1.00-1.28x on 112 of 118 kernels of two chunks a lane or more from 40 KiB on
+    (3001 x 5128 bf16 12.3 -> 10.8 us), softmax 1.00-1.11x on 74 of 78 of three or more from 80 KiB on
+    (2048 x 84936 135 -> 124); with two chunks, or (in the caches) on less, 2-9 % behind.  Rows with a half
+    vector have more to do at their ends: RMSNorm 1.00-1.10x on 77 of 77 from 80 KiB on, softmax
+    1.06x on the average from 150 KiB and five chunks or 300 KiB and three on; on smaller inputs,
+    which are one short round, 3-8 % behind.  A chunk more for the rows that start late in their line
+    costs half-vector rows 1-9 % unless it is one of many."""
+    if cfg.mode != "reg" or cfg.vec != 8 or cfg.threads_per_row % WAVE or N * 2 % LINE == 0:
+        return False
+    chunks, mib = num_chunks(cfg, N), M * N * 2 / 2**20
+    longer = num_chunks(cfg, N + (60 if cfg.half else 56))
+    if cfg.half:
+        if longer > chunks and chunks < 9:
+            return False
+        if op == "softmax":
+            worth = (mib >= 37.5 and chunks >= 5) or (mib >= 75 and chunks >= 3)
+        else:
+            worth = mib >= 20 and chunks >= 2
+    else:
+        worth = (mib >= 20 and chunks >= 3) if op == "softmax" else (mib >= 10 and chunks >= 2)
+    if not worth or longer == chunks:
+        return worth
+    padded = longer * cfg.threads_per_row * cfg.vec
+    return (longer <= 32 and use_lean(cfg, padded, op) == use_lean(cfg, N, op)
+            and _fits(regs_per_thread(cfg, padded, op), cfg.threads))
+
+
 def regs_per_thread(cfg: RowConfig, N: int, op: str) -> int:
     """Estimate of the form that gets compiled (plain, lean or online)."""
     if use_online(cfg, N, op):
@@ -188,6 +223,8 @@ def make_rowwise(
         defines["DECA_LEAN"] = 1
     if use_online(cfg, N, op):  # (which keeps no more than the lean form does)
         defines["DECA_ONLINE"] = 1
+    if use_lines(cfg, M, N, op):
+        defines["DECA_LINES"] = 1
     if cfg.half:
         defines["DECA_HALF"] = 1
     return make_spec(

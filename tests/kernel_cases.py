@@ -1,6 +1,8 @@
 """Kernel specialisations the GPU tests use, listed in one place so that the
 build step can compile all of them ahead of the GPU run."""
 
+from dataclasses import replace
+
 from deca_amd.kernels.flash_attn_hip import FAConfig, make_flash_attn_fwd
 from deca_amd.kernels.gemm_hip import GemmConfig, make_gemm_tc
 from deca_amd.kernels.rowwise_hip import RowConfig, make_rowwise
@@ -75,6 +77,39 @@ ROWWISE_ONLINE_CASES = [
     ("softmax", 6, 131072, "float16", RowConfig(1024, 1, 8, hint=True)),
 ]
 
+# Rows that are no whole number of memory lines, in chunks that start with a line: ends in the first
+# and the last wave, a last vector that is a half, a chunk more for the rows that start late in their
+# line, rows of one wave and of sixteen, several a workgroup, lean and online.  (Such rows have the
+# form in large inputs only: `lines_spec`.)
+ROWWISE_LINES_CASES = [
+    ("rmsnorm", 24, 568, "float16", RowConfig(64, 1, 8, hint=True)),
+    ("rmsnorm", 24, 580, "bfloat16", RowConfig(64, 2, 8, hint=True, half=True)),
+    ("rmsnorm", 24, 1000, "bfloat16", RowConfig(64, 2, 8)),
+    ("softmax", 24, 1032, "float16", RowConfig(64, 1, 8)),
+    ("softmax", 24, 1156, "bfloat16", RowConfig(64, 4, 8, hint=True, half=True)),
+    ("softmax", 24, 2040, "float16", RowConfig(64, 2, 8, hint=True)),
+    ("rmsnorm", 24, 1028, "float16", RowConfig(64, 4, 8, half=True)),
+    ("rmsnorm", 24, 4104, "float16", RowConfig(512, 2, 8, hint=True)),
+    ("softmax", 24, 5128, "float16", RowConfig(256, 2, 8, hint=True)),
+    ("softmax", 24, 5124, "float16", RowConfig(256, 1, 8, hint=True, half=True)),
+    ("rmsnorm", 33, 5124, "float16", RowConfig(64, 1, 8, hint=True, half=True)),
+    ("rmsnorm", 24, 5116, "float16", RowConfig(64, 1, 8, hint=True, half=True)),
+    ("rmsnorm", 24, 16388, "bfloat16", RowConfig(1024, 1, 8, hint=True, half=True)),
+    ("softmax", 24, 32760, "bfloat16", RowConfig(256, 1, 8, hint=True)),
+    ("rmsnorm", 16, 57336, "float16", RowConfig(512, 1, 8, hint=True)),
+    ("rmsnorm", 16, 128228, "bfloat16", RowConfig(1024, 1, 8, hint=True, half=True)),
+    ("softmax", 16, 126968, "float16", RowConfig(512, 1, 8, hint=True)),
+    ("softmax", 16, 114684, "bfloat16", RowConfig(1024, 1, 8, hint=True, half=True)),
+]
+
+
+def lines_spec(op, M, N, dtype, cfg, eps: float = 1e-6):
+    """The kernel of a large input, for few rows."""
+    large = dict(make_rowwise(op, 40_000_000 // N, N, dtype, RowConfig(**{**cfg.as_dict(), "rows_per_block": 1})).defines)
+    spec = make_rowwise(op, M, N, dtype, cfg, eps)
+    return replace(spec, defines=tuple(sorted({**dict(spec.defines), "DECA_LINES": large["DECA_LINES"]}.items())))
+
+
 # Full-size benchmark shapes (property checks + a sampled comparison).
 ROWWISE_FULL = [
     ("softmax", 16384, 4096, "float16", RowConfig(128, 1, 8)),
@@ -85,7 +120,8 @@ ROWWISE_FULL = [
 
 def rowwise_specs(eps: float = 1e-6):
     return [make_rowwise(op, M, N, dt, cfg, eps)
-            for op, M, N, dt, cfg in ROWWISE_CASES + ROWWISE_ONLINE_CASES + ROWWISE_FULL]
+            for op, M, N, dt, cfg in ROWWISE_CASES + ROWWISE_ONLINE_CASES + ROWWISE_FULL] \
+        + [lines_spec(*c, eps) for c in ROWWISE_LINES_CASES]
 
 
 # (M, N, K, cfg): sizes the CPU checker finishes in seconds
