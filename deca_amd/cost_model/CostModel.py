@@ -675,6 +675,11 @@ FA_TIME = {
     # workgroups share a CU); under the mask, exponent that joins the sum of the work and the
     # longest row of it
     "round": 0.636, "round_shared": -0.076, "causal": 2.73,
+    # workgroups that split keys and do not all have room at once, with rings of one slot and of more,
+    # of which fewer fit (not of the fit: with them 35 of the 357 shapes are more than 10 % off
+    # instead of 41, and the 25 choices that change on 500 others take 5.6 % more than the better of
+    # the two forms on the average instead of 11 %)
+    "split_waits": 1.02, "split_waits_slots": 1.12,
     # memory: bytes at 6.4 TB/s times this, joined by this exponent; the launch
     "memory": 1.19, "memory_join": 1.5, "launch": 0.732,
 }
@@ -724,9 +729,9 @@ def fa_time(cfg, arch, shape, causal: bool = False) -> float:
     path, and somewhat longer where two of them are close.  All workgroups at once if they fit the
     CUs; else rounds of those that do, of which a part-filled last one costs more than its share;
     under the causal mask the sum of the work or the longest row, which starts first.
-    Of the 357 shapes the first choice by it is 3.0 % behind the best measured one on the average,
-    12 of them more than 16 % (39 % at most); with three quarters of the shapes in the fit 2.8 %
-    there and 3.5 % on the others.  By `fa_score`, which prices rounds of workgroups as if they kept
+    Of the 357 shapes the first choice of `rank_fa_configs` is 3.1 % behind the best measured one on the
+    average, 18 of them more than 16 % (39 % at most); with three quarters of the shapes in the fit
+    the time was 2.8 % off there and 3.5 % on the others.  By `fa_score`, which prices rounds of workgroups as if they kept
     in step and knows no query edge, it is 7.4 % (80 % at most; 15 % from 8 rows of 32 queries per
     CU on)."""
     from deca_amd.kernels.flash_attn_hip import query_tiles
@@ -773,6 +778,8 @@ def fa_time(cfg, arch, shape, causal: bool = False) -> float:
         if most > fit:
             t *= ((1.0 - c["round"]) * rounds + c["round"] * math.ceil(rounds)
                   + c["round_shared"] * (fit > 1))
+    if split and most > fit:
+        t *= c["split_waits" if cfg.stages == 1 else "split_waits_slots"]
     memory = c["memory"] * 2 * B * H * D * 2 * (S_q + S_kv) / 6.4e6
     m = c["memory_join"]
     return (t**m + memory**m) ** (1 / m) + c["launch"]
@@ -784,8 +791,8 @@ def rank_fa_configs(configs, arch, shape, causal: bool = False, top_n: int | Non
 
     Whether the waves should split the keys (`kv_split`) is the choice where the two models differ
     most and each knows something: where `fa_score` puts such a form first its time counts 0.88,
-    else 1.06 (mean distance to the best measured form 3.2 % either way without the factors and
-    with them, but choices that were right before stay; with 1.15 one shape is 76 % off)."""
+    else 1.06 (level with no factors on the average, but choices that were right before stay; with
+    0.86 or 1.15 one shape is 76 % off)."""
     if shape[4] in (64, 128):
         whole = [c for c in configs if not getattr(c, "edge", False)]
         split_first = whole and max(whole, key=lambda c: fa_score(c, arch, shape, causal)).kv_split
