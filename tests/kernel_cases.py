@@ -102,6 +102,21 @@ ROWWISE_LINES_CASES = [
     ("softmax", 16, 114684, "bfloat16", RowConfig(1024, 1, 8, hint=True, half=True)),
 ]
 
+# Softmax of rows of every kind (masked, large, few live elements) where part of a row's vectors lie at
+# its ends: one wave to sixteen, whole and half last vectors, lean and online.  Each in the form of a
+# small input and, where it has another, in that of a large one.
+SOFTMAX_ROW_CASES = [
+    (8, 1032, "float16", RowConfig(64, 1, 8)),
+    (8, 1156, "bfloat16", RowConfig(64, 4, 8, hint=True, half=True)),
+    (8, 5128, "float16", RowConfig(128, 2, 8, hint=True)),
+    (8, 5124, "float16", RowConfig(256, 1, 8, hint=True, half=True)),
+    (8, 32760, "bfloat16", RowConfig(256, 1, 8, hint=True)),
+    (8, 57348, "float16", RowConfig(512, 2, 8, half=True)),
+    (8, 84936, "bfloat16", RowConfig(1024, 1, 8, hint=True)),
+    (8, 128252, "float16", RowConfig(1024, 1, 8, hint=True, half=True)),
+    (8, 126968, "float16", RowConfig(512, 1, 8, hint=True)),
+]
+
 
 def lines_spec(op, M, N, dtype, cfg, eps: float = 1e-6):
     """The kernel of a large input, for few rows."""
@@ -121,7 +136,8 @@ ROWWISE_FULL = [
 def rowwise_specs(eps: float = 1e-6):
     return [make_rowwise(op, M, N, dt, cfg, eps)
             for op, M, N, dt, cfg in ROWWISE_CASES + ROWWISE_ONLINE_CASES + ROWWISE_FULL] \
-        + [lines_spec(*c, eps) for c in ROWWISE_LINES_CASES]
+        + [lines_spec(*c, eps) for c in ROWWISE_LINES_CASES] \
+        + [f("softmax", *c, eps) for c in SOFTMAX_ROW_CASES for f in (make_rowwise, lines_spec)]
 
 
 # (M, N, K, cfg): sizes the CPU checker finishes in seconds
