@@ -249,10 +249,14 @@ deca_main(const elem_t* __restrict__ x,
   // chunks that lie in the row for every lane
   auto inner = [&](int c) __attribute__((always_inline)) { return c >= C_FIRST && c < C_FULL; };
   const unsigned lane_off = t * (VEC * 2) - skip;
-  const unsigned inner_off = lane_off + C_FIRST * (SPAN * 2);
+  unsigned inner_off = lane_off + C_FIRST * (SPAN * 2);
+#if DECA_LINES
+  asm volatile("" : "+v"(inner_off));  // (opaque, as below)
+#endif
   const unsigned wave_off = __builtin_amdgcn_readfirstlane(wr) * (64 * VEC * 2) - skip;
-  // Offset of a vector of a chunk at an end of the row.  (Opaque: the sum must wrap in the register
-  // and not be split into the instruction's own offset.)
+  // Offset of a vector of a chunk at an end of the row.  (Opaque: a sum that wraps does so in the
+  // register.  Split, the instruction's own offset would be added to a register that lies before the
+  // row; what the range check makes of that is not relied on.)
   auto end_off = [&](int c) __attribute__((always_inline)) {
     unsigned off = lane_off + c * (SPAN * 2);
     asm volatile("" : "+v"(off));

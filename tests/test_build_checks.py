@@ -1,5 +1,7 @@
 """The build step checks what a kernel spec promises about its generated code."""
 
+import subprocess
+
 import pytest
 
 from deca_amd.kernels.build import build_kernel, check_generated_code
@@ -93,3 +95,19 @@ def test_checked_kernels_are_tied_to_the_validated_compiler(monkeypatch):
         build.build_kernel(spec, None, "/nonexistent/never_written.hsaco".replace("/nonexistent", "/tmp"))
     monkeypatch.setenv("DECA_ALLOW_UNCHECKED_HIPCC", "1")
     build.require_validated_hipcc(spec)
+
+
+def test_no_offset_of_a_row_wraps_outside_the_register(tmp_path):
+    """Rows in chunks that start with a memory line, 64 lanes: the second chunk's offset from a lane
+    before the row is formed in the register, with none of it left to the instruction."""
+    from deca_amd.kernels.build import BASE_OPTIONS, hipcc_path
+    from deca_amd.kernels.rowwise_hip import RowConfig, make_rowwise
+
+    spec = make_rowwise("softmax", 80000, 1032, "float16", RowConfig(64, 1, 8))
+    assert ("DECA_LINES", 1) in spec.defines
+    out = tmp_path / "k.s"
+    subprocess.run([hipcc_path(), "-S", "--cuda-device-only", "--offload-arch=gfx950", *BASE_OPTIONS,
+                    *spec.options, *spec.define_flags(), spec.source_path, "-o", str(out)],
+                   check=True, capture_output=True)
+    rows = [line for line in out.read_text().splitlines() if "\tbuffer_load" in line or "\tbuffer_store" in line]
+    assert len(rows) == 6 and not any("offset:" in line for line in rows)
