@@ -63,7 +63,7 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     - non-temporal accesses: streamed data does not displace lines in L2 /
       Infinity Cache and the writes drain earlier (measured: ~8% on MI355X)
     """
-    from deca_amd.kernels.rowwise_hip import num_chunks, use_lines, use_online
+    from deca_amd.kernels.rowwise_hip import num_chunks, use_online
 
     wgs = rowwise_occupancy(cfg, arch, op, N)
     chunks = num_chunks(cfg, N)
@@ -76,6 +76,9 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     # waves meet in a reduction, fewer leave a SIMD idle).  59 shapes of 45 to 300 KiB per CU: mean
     # distance to the best 2.3 % (2.9 % in the caches) against 5.2 and 7.4 % by the terms below; longer
     # softmax rows, whose waves have twice the arithmetic of RMSNorm, gain nothing beyond 140 KiB.
+    # Rows of half vectors by the same terms (a price on the row ends that one wave has to patch put
+    # two waves or 8-byte accesses first on 90 of 1500 such shapes: over 60 of them 4 % slower on the
+    # average, -9 ... +17 %).
     rows_per_cu = M / arch.sm_nums
     kib_per_cu = rows_per_cu * N * type_size / 1024
     one_round = (cfg.mode == "reg" and cfg.threads_per_row >= arch.warp_size
@@ -112,10 +115,6 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
         rows = 1.0 / (1.0 + 0.015 * math.log2(cfg.rows_per_block))
         waves_per_cu = rows_per_cu * waves_per_row
         reduce = 1.0 / (1.0 + 0.07 * abs(math.log2(waves_per_cu / 10.5)))
-        if cfg.half and waves_per_row == 1 and use_lines(cfg, M, N, op):
-            # both ends of the row are the one wave's to patch (RMSNorm fp16 3001 x 5124: 10.5 us, and
-            # 9.9 with two waves)
-            reduce *= 0.9
     online = use_online(cfg, N, op)
     if online:
         # The first pass is done when the last chunk arrives: what lengthens the others' series of

@@ -31,6 +31,13 @@ ROWWISE = [
     ("softmax", 11580, 1648, "tpr=16,rpb=4,vec=8,mode=reg,hint=1", 17.0, 14.6),
     ("rmsnorm", 4300, 3328, "tpr=64,rpb=2,vec=4,mode=reg,hint=1", 13.1, 10.6),
     ("rmsnorm", 5950, 3448, "tpr=32,rpb=2,vec=8,mode=reg,hint=1", 17.7, 16.2),
+    # ... but what it gains there is not lost on the half vectors at the ends of its row
+    ("rmsnorm", 6760, 2460, "tpr=64,rpb=2,vec=4,mode=reg,hint=1", 14.9, 13.7),
+    ("rmsnorm", 7631, 1596, "tpr=64,rpb=1,vec=4,mode=reg,hint=1", 11.4, 10.8),
+    ("rmsnorm", 3027, 6932, "tpr=512,rpb=1,vec=4,mode=reg,hint=1", 17.6, 15.1),
+    ("rmsnorm", 3982, 4436, "tpr=256,rpb=2,vec=8,mode=reg,hint=1,half=1", 14.6, 14.0),
+    ("rmsnorm", 2439, 7132, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 14.7, 12.9),
+    ("rmsnorm", 3421, 3812, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 11.6, 10.1),
 ]
 
 
