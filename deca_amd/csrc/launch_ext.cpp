@@ -60,4 +60,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__launch() { return PyModule_Create(&module); }
+// TORCH: the version whose structures `launch` reads; the caller compares it with the one it runs with.
+PyMODINIT_FUNC PyInit__launch() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "TORCH", DECA_TORCH) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

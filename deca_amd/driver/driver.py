@@ -11,7 +11,9 @@ binding replaces `tvm.runtime.load_module(path)["main"]`
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
+import warnings
 from ctypes import POINTER, byref, c_char, c_char_p, c_float, c_int, c_size_t, c_uint, c_void_p
 
 from deca_amd.driver.build_lib import EXT_PATH, LIB_PATH
@@ -230,22 +232,26 @@ def get_driver() -> HipDriver:
     return _driver
 
 
+@functools.lru_cache(maxsize=None)
 def _load_launch():
-    """`_launch.launch` of the extension module, None where there is no torch (whose tensors it
-    takes): then only the pointer interface of this file works."""
+    """`launch` of the extension module `_launch`; None, and calls go through this file's own checks
+    and the general entry, where it is not built, or for another torch than the one that runs (whose
+    structures it reads), or there is no torch at all."""
     try:
-        import torch  # noqa: F401
+        import torch
     except ImportError:
         return None
-    if not os.path.exists(EXT_PATH):
-        raise RuntimeError(
-            f"{EXT_PATH} is missing: build it with `python -m deca_amd.driver.build_lib`")
-    from deca_amd._launch import launch
-
-    return launch
-
-
-_launch = None  # set with the first kernel that is loaded (torch is not imported before)
+    try:
+        from deca_amd import _launch as ext
+    except ImportError as err:
+        why = str(err)
+    else:
+        if ext.TORCH == torch.__version__:
+            return ext.launch
+        why = f"built for torch {ext.TORCH}, this is {torch.__version__}"
+    warnings.warn(f"{os.path.basename(EXT_PATH)}: {why}; calls of kernels take a few microseconds more until it is "
+                  "built with `python -m deca_amd.driver.build_lib`", RuntimeWarning, stacklevel=2)
+    return None
 
 
 class KernelRejected(RuntimeError):
@@ -266,14 +272,12 @@ class LoadedKernel:
         self.launches = 0  # launches issued through this object so far
         self.drv = get_driver()
         self.drv.init(device)
-        global _launch
-        if _launch is None:
-            _launch = _load_launch()
+        self._launch = _load_launch()  # (torch is not imported before the first kernel is loaded)
         self.mod = self.drv.module_load(path)
         self.fn = self.drv.get_function(self.mod, spec.symbol)
         # every kernel of this package takes at most four pointers (`launch` takes any)
         self._plan, self._plan_address = None, 0
-        if _launch is not None and 1 <= spec.nargs <= LaunchPlan.MAX_ARGS:
+        if self._launch is not None and 1 <= spec.nargs <= LaunchPlan.MAX_ARGS:
             self._plan = LaunchPlan(self.fn, spec.grid, spec.block, spec.lds_bytes, spec.nargs)
             self._plan_address = ctypes.addressof(self._plan)
         if spec.lds_bytes > 64 * 1024:
@@ -313,11 +317,11 @@ class LoadedKernel:
     def __call__(self, *tensors):
         # The host's share of a launch: 3.9 us with the checks in Python and a foreign-function
         # call, 3.2 with both in one C function, of which the runtime's own launch takes 2.7
-        # (softmax 256 x 1024, whose kernel takes 2.1: 4.3 -> 3.1 us a call; GEMM 1024^3
-        # 5.5 -> 4.4, bound by its kernel).
+        # (softmax 256 x 1024, whose kernel takes 2.1: 4.3 -> 3.2 us a call; GEMM 1024^3 takes 5.5
+        # either way).
         self.launches += 1
         if self._plan_address:
-            code = _launch(self._plan_address, *tensors)
+            code = self._launch(self._plan_address, *tensors)
             if code == 0:
                 return
             if code > 0:

@@ -3,6 +3,7 @@ checks in Python."""
 
 import ctypes
 import os
+import sys
 
 import pytest
 import torch
@@ -39,6 +40,39 @@ def test_arguments_it_cannot_take_launch_nothing(launch):
         launch(0, t, t)
     with pytest.raises(TypeError):
         launch("plan", t, t)
+
+
+def test_an_extension_that_cannot_serve_is_left_aside(launch, monkeypatch):
+    """Not built, or built for another torch: `None` and a warning, no error."""
+    from deca_amd.driver import driver
+
+    load = driver._load_launch.__wrapped__
+    assert load() is launch
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "0.1")
+        with pytest.warns(RuntimeWarning, match="built for torch"):
+            assert load() is None
+    with monkeypatch.context() as m:
+        m.delattr(sys.modules["deca_amd"], "_launch", raising=False)
+        m.setitem(sys.modules, "deca_amd._launch", None)
+        with pytest.warns(RuntimeWarning, match="take a few microseconds more"):
+            assert load() is None
+
+
+@pytest.mark.gpu
+def test_a_kernel_is_called_without_the_extension_too(monkeypatch):
+    from deca_amd.driver import driver
+    from deca_amd.kernels.rowwise_hip import RowConfig, build_rowwise, make_rowwise
+
+    monkeypatch.setattr(driver, "_load_launch", lambda: None)
+    kern = build_rowwise(make_rowwise("softmax", 512, 4096, "float16", RowConfig(128, 1, 8)))
+    assert not kern._plan_address
+    x = torch.randn(512, 4096, device="cuda").half()
+    y = torch.zeros_like(x)
+    kern(x, y)
+    assert (y.float() - torch.softmax(x.float(), -1)).abs().max().item() <= 2e-3
+    with pytest.raises(ValueError, match="contiguous device tensors"):
+        kern(x.cpu(), y)
 
 
 @pytest.mark.gpu
