@@ -651,73 +651,104 @@ def fa_score(cfg, arch, shape, causal: bool = False) -> float:
 
 
 # Coefficients of `fa_time`, in microseconds where they are times, for head dim 128 where they are
-# multiplied by D / 128.  Least squares on the logarithm of 4834 measured times (launches back to
-# back over buffers larger than the caches) of 357 shapes: 0.5 to 120 rows of 32 queries per CU,
-# S_q 128 ... 8192, S_kv 256 ... 15104, D 64 and 128, full and causal, nearly all drawn at random;
-# the configurations near a shape's best count most.
+# multiplied by D / 128.  Fitted to 10548 measured times (launches back to back over buffers larger
+# than the caches) of 910 shapes: 1 to 124 rows of 32 queries per CU, S_q 128 ... 16384, S_kv 256 ...
+# 16384, D 64 and 128, full and causal: least squares on the logarithm of the times, the
+# configurations near a shape's best counting most, and what the first choice loses on the best.
 FA_TIME = {
     # one 32 x 32 block of scores in a wave's own chain of instructions (matrix and vector part),
-    # and its share of a SIMD that has other waves to fill the gaps
-    "chain_mfma": 0.36, "chain_valu": 0.0417, "busy_mfma": 0.185, "busy_valu": 0.123,
-    # of one key step: barrier and first fragments (workgroups of eight waves need a tenth of
-    # it), the wait for a tile in a one-slot ring, and of that where waves split the keys
-    "step": 0.145, "step_8_waves": 0.2, "one_slot": 0.381, "one_slot_split": 0.0664,
-    # a 32-key tile on the CU's load path; per wave where waves split the keys
-    "load": 0.109, "load_split": 0.15,
-    "overlap": 2.2,  # exponent that joins chain, busy pipes and load path into a step's time
-    # per workgroup: fixed, per 32 query rows of a wave, per 32 keys of a tile (the first one is
-    # waited for), without a second workgroup beside it (per wave), and the meeting of the waves
-    # that split keys (per wave; less under the mask); more where more workgroups share the CU
-    "wg": 0.379, "wg_rows": 2.22, "wg_tile": 0.2, "wg_alone": 0.362,
-    "meet": 0.25, "meet_causal": -0.305, "wg_shared": 0.254, "meet_shared": 0.208,
-    # a part-filled last round counts for this share of a round (a little less where several
-    # workgroups share a CU); under the mask, exponent that joins the sum of the work and the
-    # longest row of it
-    "round": 0.636, "round_shared": -0.076, "causal": 2.73,
-    # workgroups that split keys and do not all have room at once, with rings of one slot and of more,
-    # of which fewer fit (not of the fit: with them 35 of the 357 shapes are more than 10 % off
-    # instead of 41, and the 25 choices that change on 500 others take 5.6 % more than the better of
-    # the two forms on the average instead of 11 %)
-    "split_waits": 1.02, "split_waits_slots": 1.12,
+    # and its share of a SIMD that has other waves to fill the gaps; of that, what a key step of a
+    # wave takes whatever its tile
+    "chain_mfma": 0.253, "chain_valu": 0.124, "busy_mfma": 0.17, "busy_valu": 0.0342, "issue": 0.0759,
+    # of one key step: the wait for a tile in a one-slot ring, and of that where waves split the keys
+    "one_slot": 0.304, "one_slot_split": 0.168,
+    # a 32-key tile on the CU's load path, per wave, where waves split the keys
+    "load_split": 0.0809,
+    "overlap": 1.29,  # exponent that joins chain, busy pipes and load path into a step's time
+    # per workgroup: per 32 query rows of a wave, per 32 keys of a tile (the first one is waited for),
+    # more where more workgroups share the CU, and without a second one beside it (per wave); the
+    # meeting of the waves that split keys (per wave), more where more workgroups share the CU
+    "wg_rows": 1.24, "wg_tile": 0.251, "wg_shared": 0.269, "wg_alone": 0.522,
+    "meet": 0.346, "meet_shared": 0.443,
+    # under the mask: exponent that joins the sum of the work and the longest row of it, and the
+    # share of its steps that the longest row is alone on its CU (all where waves split the keys);
+    # of both, where all workgroups fit the CUs at once; where they don't, the wait between one
+    # workgroup of a CU and the next
+    "causal": 4.48, "causal_split": 4.59, "causal_once": 3.51, "causal_split_once": 4.83,
+    "alone": 0.583, "alone_once": 0.79, "alone_split_once": 0.886, "refill": 0.783, "refill_split": 0.899,
+    # equal workgroups drift apart: a part-filled last round counts as a whole one behind the first,
+    # more and more with its share behind many
+    "drift": 0.331,
+    # PFLOP/s that the card sustains (power, and the vector work beside the matrix work), joined by
+    # this exponent
+    "rate_64": 1.08, "rate_128": 1.26, "rate_join": 4.0,
     # memory: bytes at 6.4 TB/s times this, joined by this exponent; the launch
-    "memory": 1.19, "memory_join": 1.5, "launch": 0.732,
+    "memory": 1.19, "memory_join": 1.59, "launch": 1.62,
 }
-# Logarithms of what the form of a key step does to its time; held near the medians over pairs of
-# configurations that differ in nothing else.
+# Logarithms of what the form of a key step does to its time ...
 FA_FORM = {
-    "mfma16_64": 0.0463, "mfma16_128": 0.0931, "mfma16_slots": 0.0946, "mfma16_causal": -0.054,
-    "mfma16_roll": -0.0271, "slots_causal": -0.0577, "trust_causal": 0.0693, "trust_mfma16_64": -0.0515,
-    "three_slots": 0.135, "three_slots_64": -0.046, "three_slots_large": 0.03,
-    "q_lds": 0.0982, "q_lds_64": -0.0584, "spread": 0.0146, "spread_slots": -0.116,
-    "spread_slots_64": 0.0794, "edge": -0.0406, "two_waves": 0.0582, "split_8": 0.0679,
-    "split_8_causal": 0.059,
+    "mfma16_64": 0.113, "mfma16_128": 0.122, "mfma16_slots": 0.0982, "mfma16_causal": -0.0257,
+    "mfma16_roll": -0.102, "slots": -0.162, "slots_64": 0.0705, "slots_64_causal": 0.0237,
+    "ahead": 0.0939, "trust": -0.0197, "trust_causal": 0.116, "trust_mfma16_64": -0.12,
+    "three_slots": 0.277, "three_slots_64": -0.167, "q_lds": 0.146, "q_lds_64": -0.0854,
+    "q_lds_64_rows": 0.0246, "spread": 0.0376, "spread_slots": -0.0417, "spread_slots_64": 0.0138,
+    "spread_short": -0.0251, "roll": 0.0378, "roll_64": 0.0588, "edge": 0.00224, "two_waves": 0.161,
+    "one_wave": 0.222, "split_128": 0.111, "split_two_slots": 0.0766,
+    "split_two_slots_causal": 0.0512,
+}
+# ... and to the time that the work takes at the sustained rate ("rows": times 128 rows over those of
+# all waves, less a half).
+FA_RATE = {
+    "slots_64": 0.0236, "mfma16": -0.0858, "trust": -0.0371, "rows": 0.0777, "q_lds": 0.0608,
 }
 
 
-def fa_form_factor(cfg, D: int, causal: bool) -> float:
-    """What the form of a key step (`FA_FORM`) does to its time."""
-    f, small, full = FA_FORM, D < 128, not causal
+def fa_form_factor(cfg, D: int, causal: bool, short: bool) -> float:
+    """What the form of a key step (`FA_FORM`) does to its time; `short`: at most eight of them."""
+    f, small, full, split = FA_FORM, D < 128, not causal, cfg.kv_split
     mfma16, slots = cfg.mfma == 16, int(cfg.pipe) == 2
-    log = 0.0
+    log = f["edge"] * cfg.edge
     if mfma16:
         log += f["mfma16_64"] if small else f["mfma16_128"]
         log += f["mfma16_slots"] * slots + f["mfma16_causal"] * causal + f["mfma16_roll"] * cfg.roll
-    log += f["slots_causal"] * (slots and causal)
+    if slots:
+        log += f["slots"] + (f["slots_64"] + f["slots_64_causal"] * causal) * small
+    log += f["ahead"] * (int(cfg.pipe) == 1)
     if cfg.trust:
-        log += f["trust_causal"] * causal + f["trust_mfma16_64"] * (full and mfma16 and small)
+        log += (f["trust_causal"] if causal else f["trust"]) * (not split)
+        log += f["trust_mfma16_64"] * (full and mfma16 and small)
     if cfg.stages == 3:
-        log += (f["three_slots"] + f["three_slots_64"] * small
-                + f["three_slots_large"] * (cfg.Bc * D > 32 * 128))
+        log += f["three_slots"] + f["three_slots_64"] * small
     if cfg.q_in_smem:
-        log += f["q_lds"] + f["q_lds_64"] * small
+        log += f["q_lds"] + f["q_lds_64"] * small + f["q_lds_64_rows"] * (cfg.wave_rows > 32)
     if cfg.spread:
         log += f["spread"] + (f["spread_slots"] + f["spread_slots_64"] * small) * slots
-    log += f["edge"] * cfg.edge
-    if cfg.kv_split:
-        log += (f["split_8"] + f["split_8_causal"] * causal) * (cfg.num_warps > 4)
+        log += f["spread_short"] * short
+    if cfg.roll:
+        log += f["roll"] + f["roll_64"] * small
+    if split:
+        log += f["split_128"] * (not small)
+        log += (f["split_two_slots"] + f["split_two_slots_causal"] * causal) * (cfg.stages > 1)
     else:
-        log += f["two_waves"] * (cfg.num_warps == 2)
+        log += f["two_waves"] * (cfg.num_warps == 2) + f["one_wave"] * (cfg.num_warps == 1)
     return math.exp(log)
+
+
+def fa_sustained_us(cfg, shape, causal: bool = False) -> float:
+    """Microseconds that the matrix and vector work of a launch takes at the rate that the card sustains
+    (`FA_TIME` "rate_*", PFLOP/s, and `FA_RATE`), rows and keys that are computed for nothing included."""
+    from deca_amd.kernels.flash_attn_hip import query_tiles
+
+    B, H, S_q, S_kv, D = shape
+    scores = query_tiles(cfg, S_q) * cfg.Br * S_kv
+    if causal:  # a wave computes every tile that reaches one of its rows in full
+        wq = cfg.wave_rows
+        scores = sum(-(-min(r + wq, S_kv) // cfg.Bc) * cfg.Bc * wq for r in range(0, S_q, wq))
+    f = FA_RATE
+    log = (f["slots_64"] * (int(cfg.pipe) == 2 and D < 128) + f["mfma16"] * (cfg.mfma == 16)
+           + f["trust"] * cfg.trust + f["rows"] * (128 / (cfg.num_warps * cfg.wave_rows) - 0.5)
+           + f["q_lds"] * cfg.q_in_smem)
+    return B * H * 4.0 * D * scores / (FA_TIME["rate_64" if D < 128 else "rate_128"] * 1e9) * math.exp(log)
 
 
 def fa_time(cfg, arch, shape, causal: bool = False) -> float:
@@ -726,13 +757,14 @@ def fa_time(cfg, arch, shape, causal: bool = False) -> float:
     A workgroup is a number of key steps and a fixed part.  A step takes as long as its wave's own
     chain of instructions, or as the busy pipes of a SIMD that its waves share, or as the CU's load
     path, and somewhat longer where two of them are close.  All workgroups at once if they fit the
-    CUs; else rounds of those that do, of which a part-filled last one costs more than its share;
-    under the causal mask the sum of the work or the longest row, which starts first.
-    Of the 357 shapes the first choice of `rank_fa_configs` is 3.1 % behind the best measured one on the
-    average, 18 of them more than 16 % (39 % at most); with three quarters of the shapes in the fit
-    the time was 2.8 % off there and 3.5 % on the others.  By `fa_score`, which prices rounds of workgroups as if they kept
-    in step and knows no query edge, it is 7.4 % (80 % at most; 15 % from 8 rows of 32 queries per
-    CU on)."""
+    CUs; else whole rounds of those that do (equal workgroups end together: 1.2 rounds take two) and
+    a last one of those that are left, fewer a CU and so faster; under the causal mask the sum of the
+    work or the longest row, which starts first.  Long sequences come to the rate that the card
+    sustains.
+    Over 1186 sets of configurations of a shape measured in turn (910 shapes) the first choice of
+    `rank_fa_configs` is 1.6 % behind the best on the average, more than 10 % on 47 and 39 % at most;
+    fitted to three quarters of them, 1.7 % on the others.  By `fa_score` (without the query edge) it
+    is 11 % behind, more than 10 % on 482."""
     from deca_amd.kernels.flash_attn_hip import query_tiles
 
     c = FA_TIME
@@ -741,62 +773,57 @@ def fa_time(cfg, arch, shape, causal: bool = False) -> float:
     grid = query_tiles(cfg, S_q) * B * H
     fit, _ = fa_occupancy(cfg, arch, D, grid)
     per_cu = grid / arch.sm_nums
-    most = math.ceil(per_cu)
-    together = min(most, fit)
+    together = min(math.ceil(per_cu), fit)
     mq, bc = cfg.wave_rows / 32, cfg.Bc / 32
     steps = math.ceil(S_kv / (cfg.Bc * cfg.num_warps)) if split else S_kv / cfg.Bc
-    form = fa_form_factor(cfg, D, causal)
+    share = 0.5 * (1.0 + cfg.Br / S_q) if causal else 1.0  # of the keys that the mean row sees
+    form = fa_form_factor(cfg, D, causal, steps * share <= 8)
     one_slot = c["one_slot_split" if split else "one_slot"] * (cfg.stages == 1)
 
     def step(workgroups):
         waves = workgroups * cfg.num_warps / arch.simds_per_cu
         # (a single round is as long as its fullest SIMD)
         waves = max(1.0, math.ceil(waves) if per_cu <= fit and workgroups > 1 else waves)
-        chain = (mq * bc * (c["chain_mfma"] * d + c["chain_valu"])
-                 + c["step"] * (c["step_8_waves"] if cfg.num_warps > 4 else 1.0) + one_slot)
-        busy = waves * mq * bc * (c["busy_mfma"] * d + c["busy_valu"])
-        load = (c["load_split"] * cfg.num_warps if split else c["load"]) * workgroups * bc * d
+        chain = mq * bc * (c["chain_mfma"] * d + c["chain_valu"]) + one_slot
+        busy = waves * (mq * bc * (c["busy_mfma"] * d + c["busy_valu"]) + c["issue"])
+        load = c["load_split"] * cfg.num_warps * workgroups * bc * d if split else 0.0
         p = c["overlap"]
         return (chain**p + busy**p + load**p) ** (1 / p) * form
 
-    fixed = c["wg"] + c["wg_rows"] * mq * d
-    fixed += c["meet"] * cfg.num_warps * d * mq if split else c["wg_tile"] * bc * d
-    fixed *= 1.0 + c["meet_shared" if split else "wg_shared"] * (together - 1)
-    if fit == 1 and most > 1 and not split:
-        fixed += c["wg_alone"] * cfg.num_warps * d
-    if split and causal:
-        fixed += c["meet_causal"]
-    rounds = per_cu / together
+    def fixed(workgroups):
+        t = c["wg_rows"] * mq * d + (c["meet"] * cfg.num_warps * d * mq if split else c["wg_tile"] * bc * d)
+        t *= 1.0 + c["meet_shared" if split else "wg_shared"] * (workgroups - 1)
+        return t + c["wg_alone"] * cfg.num_warps * d * (fit == 1 and per_cu > 1 and not split)
+
     if causal:
-        mean = steps * 0.5 * (1.0 + cfg.Br / S_q) * step(together) + fixed
-        longest = steps * 0.5 * (step(1) + step(together)) + fixed
-        q = c["causal"]
-        t = ((rounds * mean) ** q + longest**q) ** (1 / q)
+        mean = steps * share * step(together) + fixed(together)
+        kind = ("_split" if split else "") + ("_once" if per_cu <= fit else "")
+        alone = c.get("alone" + kind, 1.0)
+        longest = steps * (alone * step(1) + (1.0 - alone) * step(together)) + fixed(together)
+        q = c["causal" + kind]
+        t = ((per_cu / together * mean) ** q + longest**q) ** (1 / q)
+        if per_cu > fit:
+            t += c["refill" + kind]
     else:
-        t = steps * step(together) + fixed
-        if most > fit:
-            t *= ((1.0 - c["round"]) * rounds + c["round"] * math.ceil(rounds)
-                  + c["round_shared"] * (fit > 1))
-    if split and most > fit:
-        t *= c["split_waits" if cfg.stages == 1 else "split_waits_slots"]
+        rounds = math.floor(per_cu / together + 1e-9) if per_cu > fit else 1
+        whole = steps * step(together) + fixed(together)
+        t = rounds * whole
+        left = math.ceil(per_cu - rounds * together - 1e-9)
+        if left > 0:
+            apart = 1.0 - 1.0 / (1.0 + c["drift"] * (rounds - 1))
+            t += steps * step(left) + fixed(left)
+            t = (1.0 - apart) * t + apart * per_cu / together * whole
+    j, m = c["rate_join"], c["memory_join"]
+    t = (t**j + fa_sustained_us(cfg, shape, causal) ** j) ** (1 / j)
     memory = c["memory"] * 2 * B * H * D * 2 * (S_q + S_kv) / 6.4e6
-    m = c["memory_join"]
     return (t**m + memory**m) ** (1 / m) + c["launch"]
 
 
 def rank_fa_configs(configs, arch, shape, causal: bool = False, top_n: int | None = None):
     """Sort FlashAttention configs, best first: by `fa_time` at the head dims it was fitted for
-    (64 and 128), by `fa_score` at others.
-
-    Whether the waves should split the keys (`kv_split`) is the choice where the two models differ
-    most and each knows something: where `fa_score` puts such a form first its time counts 0.88,
-    else 1.06 (level with no factors on the average, but choices that were right before stay; with
-    0.86 or 1.15 one shape is 76 % off)."""
+    (64 and 128), by `fa_score` at others."""
     if shape[4] in (64, 128):
-        whole = [c for c in configs if not getattr(c, "edge", False)]
-        split_first = whole and max(whole, key=lambda c: fa_score(c, arch, shape, causal)).kv_split
-        factor = 0.88 if split_first else 1.06
-        ranked = sorted(configs, key=lambda c: fa_time(c, arch, shape, causal) * (factor if c.kv_split else 1.0))
+        ranked = sorted(configs, key=lambda c: fa_time(c, arch, shape, causal))
     else:
         ranked = sorted(configs, key=lambda c: fa_score(c, arch, shape, causal), reverse=True)
     return ranked[:top_n] if top_n else ranked

@@ -56,6 +56,22 @@ ATTENTION = [
     (8, 8, 256, 256, 64, False, "Br=64,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 6.7, 5.9),
     (6, 16, 384, 384, 64, True, "Br=64,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 11.0, 9.6),
     (6, 8, 768, 768, 128, True, "Br=32,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 25.6, 21.9),
+    # ... and the slot loop beats the key split there that was ahead of the plain loop of its tile
+    (3, 16, 704, 704, 128, True, "Br=32,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 22.6, 20.4),
+    (1, 16, 2624, 3776, 64, False, "Br=64,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 68.2, 60.6),
+    # workgroups of eight waves that split the keys take two whole rounds for 1.2 or 1.5
+    (1, 8, 1216, 12096, 128, False, "Br=32,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 132.3, 117.2),
+    (2, 32, 192, 15104, 128, False, "Br=32,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 225.1, 215.1),
+    (1, 8, 2688, 2688, 64, True, "Br=32,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 19.6, 16.8),
+    # long sequences: what the card sustains, not what a wave's own instructions would allow
+    (2, 16, 8192, 8192, 128, False, "Br=256,Bc=64,warps=8,stages=2,q_smem=0,swz=1,pipe=2,spread=8", 934.8, 904.9),
+    (4, 16, 4096, 4096, 128, False, "Br=256,Bc=64,warps=8,stages=2,q_smem=0,swz=1,pipe=2,spread=8", 481.9, 470.6),
+    (2, 32, 8192, 8192, 64, False, "Br=128,Bc=32,warps=4,stages=2,q_smem=1,swz=1,mfma=16,roll=1,trust=1", 1176, 1038),
+    (3, 32, 3840, 3840, 64, False, "Br=128,Bc=32,warps=4,stages=2,q_smem=1,swz=1,mfma=16,roll=1,trust=1", 405.2, 358.6),
+    # tiles that reach over the end of the sequence against those that divide it
+    (31, 8, 832, 832, 128, True, "Br=64,Bc=64,warps=2,stages=2,q_smem=0,swz=1,pipe=2,mfma=16,spread=8", 108.7, 79.7),
+    (5, 32, 2368, 2368, 128, True, "Br=64,Bc=32,warps=2,stages=2,q_smem=0,swz=1,mfma=16,spread=4", 323.6, 252.4),
+    (9, 16, 2880, 2880, 64, False, "Br=64,Bc=64,warps=2,stages=2,q_smem=1,swz=1,mfma=16,spread=4,trust=1", 395.1, 303.0),
 ]
 
 
@@ -71,8 +87,7 @@ def test_attention_first_rank_is_not_the_slower_form(B, H, S_q, S_kv, D, causal,
 # of the plain form ranked first
 KEY_SPLIT = [
     (1, 16, 512, 512, 64, True), (1, 16, 512, 8192, 128, False), (4, 8, 320, 384, 64, False),
-    (1, 8, 1216, 12096, 128, False), (2, 16, 768, 768, 64, True), (3, 16, 704, 704, 128, True),
-    (1, 16, 2624, 3776, 64, False),
+    (1, 8, 1216, 12096, 128, False), (2, 16, 768, 768, 64, True),
 ]
 
 
@@ -80,6 +95,25 @@ KEY_SPLIT = [
 def test_attention_first_rank_is_the_key_split_where_it_is_ahead(B, H, S_q, S_kv, D, causal):
     shape = (B, H, S_q, S_kv, D)
     assert cm.rank_fa_configs(Solver.solve_flash_attn(ARCH, *shape), ARCH, shape, causal)[0].kv_split
+
+
+@pytest.mark.parametrize("D,causal", [(64, False), (64, True), (128, False), (128, True)])
+def test_tuning_attention_measures_the_stored_winner(D, causal):
+    """The tuning driver measures the first 16 configurations."""
+    shape = (4, 16, 4096, 4096, D)
+    stored = tuned.lookup(tuned.make_key("flash_attn", shape, causal=causal))
+    ranked = cm.rank_fa_configs(Solver.solve_flash_attn(ARCH, *shape), ARCH, shape, causal, top_n=16)
+    assert stored in ranked
+
+
+@pytest.mark.parametrize("S", [2048, 8192])
+@pytest.mark.parametrize("D,causal", [(64, False), (64, True), (128, False), (128, True)])
+def test_no_attention_time_is_below_the_sustained_rate(S, D, causal):
+    """1.25 PFLOP/s is more than any form was measured at."""
+    shape = (2, 32, S, S, D)
+    flops = 4.0 * 2 * 32 * S * S * D * (0.5 if causal else 1.0)
+    for cfg in Solver.solve_flash_attn(ARCH, *shape):
+        assert flops / cm.fa_time(cfg, ARCH, shape, causal) < 1.25e9, cfg
 
 
 @pytest.mark.parametrize("M,N,K,cfg", GEMM_EDGE_CASES, ids=lambda v: str(v))
