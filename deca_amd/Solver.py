@@ -468,7 +468,8 @@ FA_DOMAINS = {
 # such shapes the best of them was 5 ... 51 % ahead (B4 H8 S 3392 D 64: 135 -> 106 us; B9 H16 S 576
 # D 128 causal: 1.4x).  Not for multiples of 128 (tiles of 256: 4 ... 24 % behind on 6 of 8), nor below
 # the stated rows of 32 queries per CU, where the tiles are too few (0.8 ... 1.2x on six shapes), nor
-# with less than the stated share of the rows in the sequence.
+# with less than the stated share of the rows in the sequence.  (Measured at D 64 and 128; for larger
+# head dims see `rank_fa_configs`.)
 FA_EDGE_BR = (128, 256)
 FA_EDGE_MIN_FILL = 0.6
 FA_EDGE_MIN_ROWS_PER_CU = 5.25

@@ -825,5 +825,11 @@ def rank_fa_configs(configs, arch, shape, causal: bool = False, top_n: int | Non
     if shape[4] in (64, 128):
         ranked = sorted(configs, key=lambda c: fa_time(c, arch, shape, causal))
     else:
-        ranked = sorted(configs, key=lambda c: fa_score(c, arch, shape, causal), reverse=True)
+        # Query edges by the score are ahead of the first dividing tile on 45 of 46 shapes of D 192 and
+        # 384 and of full ones of D 256 and 320 (0.96 ... 6x).  Under the mask at D 256 and 320 the score
+        # does not know what their registers cost: 0.39 ... 1.02x on eight shapes of up to 576 rows,
+        # 0.86 ... 1.8x on eight from 960 on.
+        late = causal and 192 < shape[4] < 384 and shape[2] < 960
+        ranked = sorted(configs, key=lambda c: (not (late and c.edge), fa_score(c, arch, shape, causal)),
+                        reverse=True)
     return ranked[:top_n] if top_n else ranked

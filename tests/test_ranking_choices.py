@@ -72,6 +72,15 @@ ATTENTION = [
     (31, 8, 832, 832, 128, True, "Br=64,Bc=64,warps=2,stages=2,q_smem=0,swz=1,pipe=2,mfma=16,spread=8", 108.7, 79.7),
     (5, 32, 2368, 2368, 128, True, "Br=64,Bc=32,warps=2,stages=2,q_smem=0,swz=1,mfma=16,spread=4", 323.6, 252.4),
     (9, 16, 2880, 2880, 64, False, "Br=64,Bc=64,warps=2,stages=2,q_smem=1,swz=1,mfma=16,spread=4,trust=1", 395.1, 303.0),
+    (2, 16, 1344, 1344, 192, False, "Br=64,Bc=32,warps=2,stages=2,q_smem=0,swz=1,mfma=16,trust=1", 100.5, 60.7),
+    (11, 8, 2752, 2752, 192, True, "Br=64,Bc=32,warps=2,stages=2,q_smem=0,swz=1,mfma=16", 447.9, 272.8),
+    (9, 8, 1600, 1600, 256, False, "Br=64,Bc=32,warps=2,stages=2,q_smem=0,swz=1,mfma=16,trust=1", 369.2, 260.6),
+    # ... but for short causal ones of wide heads
+    (19, 32, 448, 448, 320, True, "Br=128,Bc=64,warps=4,stages=2,q_smem=0,swz=1,pipe=2,mfma=16,spread=8,edge=1",
+     578.6, 224.5),
+    (20, 32, 576, 576, 320, True, "Br=128,Bc=64,warps=4,stages=2,q_smem=0,swz=1,pipe=2,mfma=16,spread=8,edge=1",
+     855.1, 337.1),
+    (23, 16, 576, 576, 256, True, "Br=256,Bc=32,warps=8,stages=1,q_smem=1,swz=1,mfma=16,edge=1", 187.7, 156.7),
 ]
 
 

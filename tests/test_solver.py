@@ -261,6 +261,26 @@ def test_flash_attn_rolled_loop_is_offered_where_registers_are_tight():
         fa.check_config(fa.FAConfig(256, 64, 8, 2, pipe=2, roll=True), 4096, 4096, 128)
 
 
+@pytest.mark.parametrize("B,H,S,D,offered", [
+    (4, 8, 3392, 64, True), (9, 16, 576, 128, True), (2, 16, 1344, 192, True),
+    (4, 8, 3328, 64, False),   # tiles of 128 rows divide it
+    (1, 16, 2752, 64, True), (1, 16, 2624, 64, False),  # 5.25 rows per CU
+    (32, 32, 64, 64, False), (16, 32, 96, 64, True), (16, 32, 160, 128, True),  # share of a tile's rows
+])
+def test_flash_attn_query_edges_are_offered_inside_their_gates(B, H, S, D, offered):
+    configs = [c for c in Solver.solve_flash_attn(ARCH, B, H, S, S, D) if c.edge]
+    assert bool(configs) == offered
+    for c in configs:
+        fa.check_config(c, S, S, D)
+        assert S % c.Br and c.Br in Solver.FA_EDGE_BR and int(c.pipe) in (0, 2) and not c.kv_split
+        assert S >= Solver.FA_EDGE_MIN_FILL * fa.query_tiles(c, S) * c.Br
+        assert B * H * S // 32 >= Solver.FA_EDGE_MIN_ROWS_PER_CU * ARCH.sm_nums
+        # the same tile divides a longer sequence without the flag, and this one not at all
+        fa.check_config(replace(c, edge=False), fa.query_tiles(c, S) * c.Br, S, D)
+        with pytest.raises(AssertionError):
+            fa.check_config(replace(c, edge=False), S, S, D)
+
+
 def test_flash_attn_knobs_of_the_reference():
     """`q_in_smem`, `swizzle` and `stages` 1..3 (flash_attn_tir.py:35-38) all reach the
     kernel: LDS footprint, register estimate and the macros of the specialisation."""
