@@ -385,8 +385,8 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
   const int nkv_all = NKV;
 #endif
   const int nkv = (nkv_all - kvg + KVG - 1) / KVG;  // (a wave's share may be empty)
-  // First row of this wave, and (DECA_QEDGE) how many rows there are from it on: a row beyond the
-  // sequence is loaded as the last one again and not stored.
+  // First row of this wave.  (DECA_QEDGE: a row beyond the sequence is loaded as the last one again
+  // and not stored.)
   const int q_row0 = qt * BR + qw * WQ;
   const int q_row0_u = qt * BR + qw_u * WQ;
   auto q_row = [&](int r) __attribute__((always_inline)) {  // row r of the wave, relative to q_row0
@@ -1369,12 +1369,14 @@ deca_main(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
 #else
   for (int j = 0; j < nkv; ++j) {
     wait_and_barrier();
-    acc_t s_acc[KT][MQ];
-    half8 pf[KK][MQ];
-    compute_s(s_acc, 0, nothing);
-    mask_s(s_acc, j);
-    softmax(s_acc, pf);
-    compute_pv(pf, 0);
+    if (!q_idle) {
+      acc_t s_acc[KT][MQ];
+      half8 pf[KK][MQ];
+      compute_s(s_acc, 0, nothing);
+      mask_s(s_acc, j);
+      softmax(s_acc, pf);
+      compute_pv(pf, 0);
+    }
     // single slot: everyone must be done reading before the refill
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
