@@ -317,8 +317,8 @@ class LoadedKernel:
     def __call__(self, *tensors):
         # The host's share of a launch: 3.9 us with the checks in Python and a foreign-function
         # call, 3.2 with both in one C function, of which the runtime's own launch takes 2.7
-        # (softmax 256 x 1024, whose kernel takes 2.1: 4.3 -> 3.2 us a call; GEMM 1024^3 takes 5.5
-        # either way).
+        # (softmax 256 x 1024, whose kernel takes 2.1: 4.3 -> 3.2 us a call; GEMM 1024^3 is bound by
+        # its kernel: 4.4 us a call on the same tensors, 5.5 over three sets of them in turn).
         self.launches += 1
         if self._plan_address:
             code = self._launch(self._plan_address, *tensors)
