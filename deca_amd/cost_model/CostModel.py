@@ -63,7 +63,7 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     - non-temporal accesses: streamed data does not displace lines in L2 /
       Infinity Cache and the writes drain earlier (measured: ~8% on MI355X)
     """
-    from deca_amd.kernels.rowwise_hip import num_chunks, use_online
+    from deca_amd.kernels.rowwise_hip import ONLINE_MIN_N, num_chunks, use_online
 
     wgs = rowwise_occupancy(cfg, arch, op, N)
     chunks = num_chunks(cfg, N)
@@ -114,7 +114,10 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
         wave_eff = math.sqrt(rows_per_cu / (math.ceil(grid / arch.sm_nums) * cfg.rows_per_block))
         rows = 1.0 / (1.0 + 0.015 * math.log2(cfg.rows_per_block))
         waves_per_cu = rows_per_cu * waves_per_row
-        reduce = 1.0 / (1.0 + 0.07 * abs(math.log2(waves_per_cu / 10.5)))
+        # (one wave a row is no more than its due where there are more rows: priced against 10.5 waves,
+        # 8-byte accesses and two waves a row came first on 65 of 4983 shapes, nearly all of 29 to 32
+        # rows per CU, and took 3.8 % longer on the average, 7.6 % in the caches)
+        reduce = 1.0 / (1.0 + 0.07 * abs(math.log2(waves_per_cu / max(10.5, rows_per_cu))))
     online = use_online(cfg, N, op)
     if online:
         # The first pass is done when the last chunk arrives: what lengthens the others' series of
@@ -140,6 +143,10 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
             ahead = N >= (4100 if softmax else 3400) and not (5200 if softmax else 6900) < N < 7900
         if ahead:
             lanes = 0.93
+    # Softmax rows of the online form's lengths: its 16-byte accesses are 1.04-1.57x ahead of 8-byte
+    # ones on 76 of 76 shapes of 1 to 6 rows per CU (of which those may fit a CU one more).
+    if op == "softmax" and N >= ONLINE_MIN_N and cfg.mode == "reg" and cfg.vec * type_size < 16:
+        lanes = 0.75
     # A workgroup that has a long row to itself leaves a CU room for two or three others, one with
     # two such rows for none (36K ... 55K elements: 10-37 % behind one row of 256 lanes on 13 of 13
     # shapes), nor do 1024 lanes (33K ... 50K: 2-42 % behind on 20 of 20; with up to 4.5 rows per CU

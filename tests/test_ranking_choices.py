@@ -31,6 +31,10 @@ ROWWISE = [
     ("softmax", 11580, 1648, "tpr=16,rpb=4,vec=8,mode=reg,hint=1", 17.0, 14.6),
     ("rmsnorm", 4300, 3328, "tpr=64,rpb=2,vec=4,mode=reg,hint=1", 13.1, 10.6),
     ("rmsnorm", 5950, 3448, "tpr=32,rpb=2,vec=8,mode=reg,hint=1", 17.7, 16.2),
+    # ... nor is one wave a row too many where there are more rows than the waves a CU needs
+    ("rmsnorm", 7496, 824, "tpr=64,rpb=2,vec=4,mode=reg,hint=1", 7.0, 6.2),
+    ("rmsnorm", 8181, 1028, "tpr=64,rpb=1,vec=4,mode=reg,hint=1", 9.2, 8.3),
+    ("softmax", 8015, 904, "tpr=64,rpb=1,vec=4,mode=reg,hint=1", 7.5, 7.1),
     # ... but what it gains there is not lost on the half vectors at the ends of its row
     ("rmsnorm", 6760, 2460, "tpr=64,rpb=2,vec=4,mode=reg,hint=1", 14.9, 13.7),
     ("rmsnorm", 7631, 1596, "tpr=64,rpb=1,vec=4,mode=reg,hint=1", 11.4, 10.8),
@@ -38,6 +42,9 @@ ROWWISE = [
     ("rmsnorm", 3982, 4436, "tpr=256,rpb=2,vec=8,mode=reg,hint=1,half=1", 14.6, 14.0),
     ("rmsnorm", 2439, 7132, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 14.7, 12.9),
     ("rmsnorm", 3421, 3812, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 11.6, 10.1),
+    # long softmax rows that 8-byte accesses fit three of into a CU, 16-byte ones two
+    ("softmax", 572, 64932, "tpr=512,rpb=1,vec=4,mode=reg,hint=1", 38.8, 29.9),
+    ("softmax", 653, 64620, "tpr=512,rpb=1,vec=4,mode=reg,hint=1", 40.3, 38.0),
 ]
 
 
