@@ -658,55 +658,55 @@ def fa_score(cfg, arch, shape, causal: bool = False) -> float:
 
 
 # Coefficients of `fa_time`, in microseconds where they are times, for head dim 128 where they are
-# multiplied by D / 128.  Fitted to 10548 measured times (launches back to back over buffers larger
-# than the caches) of 910 shapes: 1 to 124 rows of 32 queries per CU, S_q 128 ... 16384, S_kv 256 ...
+# multiplied by D / 128.  Fitted to 10936 measured times (launches back to back over buffers larger
+# than the caches) of 1024 shapes: 1 to 124 rows of 32 queries per CU, S_q 128 ... 16384, S_kv 256 ...
 # 16384, D 64 and 128, full and causal: least squares on the logarithm of the times, the
 # configurations near a shape's best counting most, and what the first choice loses on the best.
 FA_TIME = {
     # one 32 x 32 block of scores in a wave's own chain of instructions (matrix and vector part),
     # and its share of a SIMD that has other waves to fill the gaps; of that, what a key step of a
     # wave takes whatever its tile
-    "chain_mfma": 0.253, "chain_valu": 0.124, "busy_mfma": 0.17, "busy_valu": 0.0342, "issue": 0.0759,
+    "chain_mfma": 0.238, "chain_valu": 0.112, "busy_mfma": 0.162, "busy_valu": 0.0377, "issue": 0.0806,
     # of one key step: the wait for a tile in a one-slot ring, and of that where waves split the keys
-    "one_slot": 0.304, "one_slot_split": 0.168,
+    "one_slot": 0.243, "one_slot_split": 0.162,
     # a 32-key tile on the CU's load path, per wave, where waves split the keys
-    "load_split": 0.0809,
-    "overlap": 1.29,  # exponent that joins chain, busy pipes and load path into a step's time
+    "load_split": 0.0709,
+    "overlap": 1.2,  # exponent that joins chain, busy pipes and load path into a step's time
     # per workgroup: per 32 query rows of a wave, per 32 keys of a tile (the first one is waited for),
     # more where more workgroups share the CU, and without a second one beside it (per wave); the
     # meeting of the waves that split keys (per wave), more where more workgroups share the CU
-    "wg_rows": 1.24, "wg_tile": 0.251, "wg_shared": 0.269, "wg_alone": 0.522,
-    "meet": 0.346, "meet_shared": 0.443,
+    "wg_rows": 1.27, "wg_tile": 0.237, "wg_shared": 0.145, "wg_alone": 0.49,
+    "meet": 0.335, "meet_shared": 0.379,
     # under the mask: exponent that joins the sum of the work and the longest row of it, and the
     # share of its steps that the longest row is alone on its CU (all where waves split the keys);
     # of both, where all workgroups fit the CUs at once; where they don't, the wait between one
     # workgroup of a CU and the next
-    "causal": 4.48, "causal_split": 4.59, "causal_once": 3.51, "causal_split_once": 4.83,
-    "alone": 0.583, "alone_once": 0.79, "alone_split_once": 0.886, "refill": 0.783, "refill_split": 0.899,
+    "causal": 7.17, "causal_split": 4.83, "causal_once": 4.05, "causal_split_once": 4.68,
+    "alone": 0.59, "alone_once": 0.798, "alone_split_once": 0.896, "refill": 1.16, "refill_split": 0.884,
     # equal workgroups drift apart: a part-filled last round counts as a whole one behind the first,
     # more and more with its share behind many
-    "drift": 0.331,
+    "drift": 0.23,
     # PFLOP/s that the card sustains (power, and the vector work beside the matrix work), joined by
     # this exponent
-    "rate_64": 1.08, "rate_128": 1.26, "rate_join": 4.0,
+    "rate_64": 1.09, "rate_128": 1.26, "rate_join": 4.0,
     # memory: bytes at 6.4 TB/s times this, joined by this exponent; the launch
-    "memory": 1.19, "memory_join": 1.59, "launch": 1.62,
+    "memory": 1.24, "memory_join": 1.62, "launch": 1.72,
 }
 # Logarithms of what the form of a key step does to its time ...
 FA_FORM = {
-    "mfma16_64": 0.113, "mfma16_128": 0.122, "mfma16_slots": 0.0982, "mfma16_causal": -0.0257,
-    "mfma16_roll": -0.102, "slots": -0.162, "slots_64": 0.0705, "slots_64_causal": 0.0237,
-    "ahead": 0.0939, "trust": -0.0197, "trust_causal": 0.116, "trust_mfma16_64": -0.12,
-    "three_slots": 0.277, "three_slots_64": -0.167, "q_lds": 0.146, "q_lds_64": -0.0854,
-    "q_lds_64_rows": 0.0246, "spread": 0.0376, "spread_slots": -0.0417, "spread_slots_64": 0.0138,
-    "spread_short": -0.0251, "roll": 0.0378, "roll_64": 0.0588, "edge": 0.00224, "two_waves": 0.161,
-    "one_wave": 0.222, "split_128": 0.111, "split_two_slots": 0.0766,
-    "split_two_slots_causal": 0.0512,
+    "mfma16_64": 0.109, "mfma16_128": 0.122, "mfma16_slots": 0.0957, "mfma16_causal": -0.0263,
+    "mfma16_roll": -0.0994, "slots": -0.16, "slots_64": 0.0968, "slots_64_causal": 0.000893,
+    "ahead": 0.086, "trust": -0.0277, "trust_causal": 0.121, "trust_mfma16_64": -0.119,
+    "three_slots": 0.288, "three_slots_64": -0.176, "q_lds": 0.147, "q_lds_64": -0.0915,
+    "q_lds_64_rows": 0.037, "spread": 0.0378, "spread_slots": -0.0395, "spread_slots_64": 0.0165,
+    "spread_short": -0.0161, "slots_128_keys": -0.068, "plain_128_keys": 0.0566, "roll": -0.00181,
+    "roll_64": 0.108, "edge": 0.00279, "two_waves": 0.171, "one_wave": 0.241, "split_128": 0.113,
+    "split_two_slots": 0.0767, "split_two_slots_causal": 0.0483,
 }
 # ... and to the time that the work takes at the sustained rate ("rows": times 128 rows over those of
 # all waves, less a half).
 FA_RATE = {
-    "slots_64": 0.0236, "mfma16": -0.0858, "trust": -0.0371, "rows": 0.0777, "q_lds": 0.0608,
+    "slots_64": 0.0236, "mfma16": -0.0839, "trust": -0.0364, "rows": 0.0729, "q_lds": 0.0694,
 }
 
 
@@ -721,6 +721,11 @@ def fa_form_factor(cfg, D: int, causal: bool, short: bool) -> float:
     if slots:
         log += f["slots"] + (f["slots_64"] + f["slots_64_causal"] * causal) * small
     log += f["ahead"] * (int(cfg.pipe) == 1)
+    if cfg.Bc >= 128 and not split:
+        if slots:  # (level in four waves, and under the mask)
+            log += f["slots_128_keys"] * (full and cfg.num_warps != 4)
+        else:
+            log += f["plain_128_keys"]
     if cfg.trust:
         log += (f["trust_causal"] if causal else f["trust"]) * (not split)
         log += f["trust_mfma16_64"] * (full and mfma16 and small)
@@ -768,10 +773,10 @@ def fa_time(cfg, arch, shape, causal: bool = False) -> float:
     a last one of those that are left, fewer a CU and so faster; under the causal mask the sum of the
     work or the longest row, which starts first.  Long sequences come to the rate that the card
     sustains.
-    Over 1186 sets of configurations of a shape measured in turn (910 shapes) the first choice of
-    `rank_fa_configs` is 1.6 % behind the best on the average, more than 10 % on 47 and 39 % at most;
-    fitted to three quarters of them, 1.7 % on the others.  By `fa_score` (without the query edge) it
-    is 11 % behind, more than 10 % on 482."""
+    Over 1350 sets of configurations of a shape measured in turn (1024 shapes) the first choice of
+    `rank_fa_configs` is 1.5 % behind the best on the average, more than 10 % on 53 and 39 % at most;
+    fitted to three quarters of them, 1.6 % on the others.  By `fa_score` (without the query edge) it
+    is 11 % behind, more than 10 % on 565."""
     from deca_amd.kernels.flash_attn_hip import query_tiles
 
     c = FA_TIME

@@ -59,6 +59,9 @@ def test_rowwise_first_rank_is_not_the_slower_form(op, M, N, slower, slower_us, 
 ATTENTION = [
     # few keys, more than two rows of 32 queries per CU: the plain forms fill the SIMDs too
     (3, 16, 384, 384, 64, False, "Br=32,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 8.2, 7.1),
+    # (of which the slot loop of two waves takes 128 keys a step)
+    (3, 16, 384, 384, 64, False, "Br=64,Bc=64,warps=2,stages=2,q_smem=0,swz=1,pipe=2", 8.4, 7.1),
+    (3, 16, 384, 384, 64, False, "Br=64,Bc=64,warps=2,stages=2,q_smem=0,swz=1,pipe=2,spread=8", 8.4, 7.1),
     (5, 16, 384, 384, 64, False, "Br=64,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 10.5, 9.1),
     (8, 8, 256, 256, 64, False, "Br=64,Bc=32,warps=8,stages=1,q_smem=0,swz=1,kvs=1", 6.7, 5.9),
     (6, 16, 384, 384, 64, True, "Br=64,Bc=32,warps=4,stages=1,q_smem=0,swz=1,kvs=1", 11.0, 9.6),
