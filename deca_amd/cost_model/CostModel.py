@@ -63,7 +63,7 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     - non-temporal accesses: streamed data does not displace lines in L2 /
       Infinity Cache and the writes drain earlier (measured: ~8% on MI355X)
     """
-    from deca_amd.kernels.rowwise_hip import ONLINE_MIN_N, num_chunks, use_online
+    from deca_amd.kernels.rowwise_hip import ONLINE_MIN_N, num_chunks, use_lines, use_online
 
     wgs = rowwise_occupancy(cfg, arch, op, N)
     chunks = num_chunks(cfg, N)
@@ -76,9 +76,10 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
     # waves meet in a reduction, fewer leave a SIMD idle).  59 shapes of 45 to 300 KiB per CU: mean
     # distance to the best 2.3 % (2.9 % in the caches) against 5.2 and 7.4 % by the terms below; longer
     # softmax rows, whose waves have twice the arithmetic of RMSNorm, gain nothing beyond 140 KiB.
-    # Rows of half vectors by the same terms (a price on the row ends that one wave has to patch put
-    # two waves or 8-byte accesses first on 90 of 1500 such shapes: over 60 of them 4 % slower on the
-    # average, -9 ... +17 %).
+    # Both ends of a half-vector row are the one wave's to patch where a wave has it to itself: 4 %,
+    # which decides where two waves are that near (17 of 60 shapes on which a price of 10 % would: they are
+    # level there, 2 % ahead in the caches, 1787 x 7260 9.0 against 10.1 us; with 10 % the 60 are 4 %
+    # slower on the average).
     rows_per_cu = M / arch.sm_nums
     kib_per_cu = rows_per_cu * N * type_size / 1024
     one_round = (cfg.mode == "reg" and cfg.threads_per_row >= arch.warp_size
@@ -118,6 +119,8 @@ def rowwise_score(cfg, arch, op: str, M: int, N: int, type_size: int = 2) -> flo
         # 8-byte accesses and two waves a row came first on 65 of 4983 shapes, nearly all of 29 to 32
         # rows per CU, and took 3.8 % longer on the average, 7.6 % in the caches)
         reduce = 1.0 / (1.0 + 0.07 * abs(math.log2(waves_per_cu / max(10.5, rows_per_cu))))
+        if cfg.half and waves_per_row == 1 and use_lines(cfg, M, N, op):
+            reduce *= 0.96
     online = use_online(cfg, N, op)
     if online:
         # The first pass is done when the last chunk arrives: what lengthens the others' series of

@@ -42,6 +42,9 @@ ROWWISE = [
     ("rmsnorm", 3982, 4436, "tpr=256,rpb=2,vec=8,mode=reg,hint=1,half=1", 14.6, 14.0),
     ("rmsnorm", 2439, 7132, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 14.7, 12.9),
     ("rmsnorm", 3421, 3812, "tpr=128,rpb=1,vec=8,mode=reg,hint=1,half=1", 11.6, 10.1),
+    # ... where two waves a row are not nearly as good
+    ("rmsnorm", 1787, 7260, "tpr=64,rpb=1,vec=8,mode=reg,hint=1,half=1", 10.1, 9.0),
+    ("rmsnorm", 1820, 7220, "tpr=64,rpb=1,vec=8,mode=reg,hint=1,half=1", 11.0, 10.1),
     # long softmax rows that 8-byte accesses fit three of into a CU, 16-byte ones two
     ("softmax", 572, 64932, "tpr=512,rpb=1,vec=4,mode=reg,hint=1", 38.8, 29.9),
     ("softmax", 653, 64620, "tpr=512,rpb=1,vec=4,mode=reg,hint=1", 40.3, 38.0),
